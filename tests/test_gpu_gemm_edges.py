@@ -1,0 +1,88 @@
+"""GEMM operands of any extent, alignment and leading dimension.
+
+The kernels read and write 16-byte pieces at the element's own alignment,
+clamp the rows and columns of edge tiles and guard the last partial k-stage.
+Every matrix here is embedded in a larger buffer of NaN (row padding, the
+elements before its first and after its last): a piece that read past a row
+it owns, or an accumulator that took a clamped row's product, would carry a
+NaN into the result; a store past an edge would replace a NaN around D.
+Bar: the sum bound of K products in the data type, normwise (fp64 1e-12,
+fp32 1e-5, the bar of the other kernel tests)."""
+
+import pytest
+import torch
+
+from util import normwise
+
+pytestmark = pytest.mark.gpu
+TOL = {torch.float64: 1e-12, torch.float32: 1e-5}
+
+
+def embed(x, ld, off, dt):
+    """x (batch, rows, cols) in a NaN buffer: row pitch ld, first element at
+    `off`, batches ld + 1 elements apart beyond their rows. Returns the
+    buffer, the batch stride and a view of the data in it."""
+    b, r, c = x.shape
+    stride = r * ld + 1
+    buf = torch.full((off + b * stride + 8,), float("nan"), dtype=dt, device="cuda")
+    view = torch.as_strided(buf, (b, r, c), (stride, ld, 1), off)
+    view.copy_(x.to("cuda", dt))
+    return buf, stride, view
+
+
+# (M, N, K): around the 32-, 64-, 128- and 256-wide tiles and the 16-, 64- and
+# 128-deep stages; one row or column; fewer rows than a 16-byte piece holds.
+SHAPES = [(65, 129, 17), (63, 127, 33), (130, 257, 64), (64, 256, 48), (1, 70, 40), (70, 1, 40), (3, 3, 19),
+          (2, 131, 15), (129, 2, 16), (33, 31, 129), (150, 150, 55), (31, 33, 130), (200, 66, 1), (257, 513, 31)]
+
+
+@pytest.mark.parametrize("dt", [torch.float64, torch.float32])
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_gemm_unaligned_ragged(hip, dt, ta, tb, M, N, K):
+    from trntensor_amd.hip import engine
+
+    g = torch.Generator().manual_seed(M * 5 + N * 3 + K)
+    batch = 2
+    for pad, off, with_c in ((1, 1, True), (0, 0, False), (2, 3, False)):
+        A = torch.randn(batch, M, K, generator=g, dtype=torch.float64)
+        B = torch.randn(batch, K, N, generator=g, dtype=torch.float64)
+        C = torch.randn(batch, M, N, generator=g, dtype=torch.float64)
+        sa = A.transpose(1, 2) if ta else A
+        sb = B.transpose(1, 2) if tb else B
+        lda, ldb, ldc, ldd = sa.shape[2] + pad, sb.shape[2] + pad, N + pad, N + 2 * pad
+        Ab, sA, _ = embed(sa, lda, off, dt)
+        Bb, sB, _ = embed(sb, ldb, off, dt)
+        Cb, sC, _ = embed(C, ldc, off, dt)
+        Db, sD, D = embed(torch.full((batch, M, N), float("nan")), ldd, off, dt)
+        engine.gemm(ta, tb, M, N, K, Ab, lda, sA, Bb, ldb, sB, Db, ldd, sD, batch, 1.5, 0.5 if with_c else 0.0,
+                    Cb[off:] if with_c else None, ldc, sC, a_off=off, b_off=off, d_off=off)
+        ref = 1.5 * torch.bmm(A, B) + (0.5 * C if with_c else 0.0)
+        torch.cuda.synchronize()
+        assert normwise(D.cpu().double(), ref) <= TOL[dt], (pad, off)
+        assert int(torch.isnan(Db).sum()) == Db.numel() - batch * M * N, (pad, off)
+
+
+@pytest.mark.parametrize("dt", [torch.float64, torch.float32])
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("M,N,K", [(65, 129, 17), (64, 128, 32), (130, 255, 50), (5, 3, 40), (70, 2, 33), (3, 131, 16)])
+def test_gemm_dot_unaligned_ragged(hip, dt, ta, tb, M, N, K):
+    """The dot epilogue on ragged, unaligned operands: rows and columns past
+    the matrix must not enter the sum."""
+    from trntensor_amd.hip import engine
+
+    g = torch.Generator().manual_seed(M + N + K)
+    A = torch.randn(1, M, K, generator=g, dtype=torch.float64)
+    B = torch.randn(1, K, N, generator=g, dtype=torch.float64)
+    E = torch.randn(1, M, N, generator=g, dtype=torch.float64)
+    sa, sb = A.transpose(1, 2) if ta else A, B.transpose(1, 2) if tb else B
+    lda, ldb = sa.shape[2] + 1, sb.shape[2] + 1
+    Ab, sA, _ = embed(sa, lda, 1, dt)
+    Bb, sB, _ = embed(sb, ldb, 1, dt)
+    Eb, _, _ = embed(E, N + 1, 1, dt)
+    out = torch.full((), float("nan"), dtype=dt, device="cuda")
+    engine.gemm_dot(ta, tb, M, N, K, Ab, lda, sA, Bb, ldb, sB, 1, M, N, Eb[1:], [0, N + 1, 0, 1, 0], None, None,
+                    1.0, 0.0, None, out, a_off=1, b_off=1)
+    X = torch.bmm(A, B)
+    scale = float((X.abs() * E.abs()).sum())
+    assert abs(float(out) - float((X * E).sum())) <= TOL[dt] * scale

@@ -26,84 +26,120 @@ constexpr int kBK = 16;
 constexpr int kThreads = 256;
 
 
+// 16 bytes of T in memory at T's own alignment. gfx950 serves a 16-byte global
+// access at any element address, so operands, leading dimensions and batch
+// strides of any parity take the vector loads and stores; an access that is
+// not 16-byte aligned only touches one cache line more now and then.
+template <typename T>
+struct Mem16 {
+    typedef T type __attribute__((ext_vector_type(16 / sizeof(T)), aligned(sizeof(T))));
+};
+
 // One operand's ROWS x BK stage: global -> registers -> LDS, plus fragment reads.
 // KC: element (row, k) at p[row * ld + k]; otherwise at p[k * ld + row].
 // Each thread stages E = ROWS * BK / 256 elements as NC 16-byte pieces:
-//   KC: row t / (BK / E), one contiguous chunk from k = (t % (BK / E)) E;
-//   RC: 16 threads per k-row, k-rows t / 16 + 16 j; within a k-row a
-//       thread's pieces are (t % 16) + 16 c, so every instruction covers 256
-//       contiguous bytes of the k-row (coalesced loads, conflict-free stores).
+//   KC: row t / TPK; BK = 16: one contiguous chunk from k = (t % TPK) E; deeper
+//       stages: pieces (t % TPK) + TPK c, so an instruction's lanes read
+//       TPK * 16 contiguous bytes of each row;
+//   RC: TPR threads per k-row, k-rows t / TPR + (256 / TPR) j; within a k-row a
+//       thread's pieces are (t % TPR) + TPR c, so every instruction covers
+//       TPR * 16 contiguous bytes of the k-row (coalesced loads,
+//       conflict-free stores).
 // RC k-rows are padded by 4 elements: the four lane groups of a fragment read
 // (k-rows 4 g + s) then land on disjoint LDS banks.
-template <typename T, int ROWS, bool KC, bool VEC, int BK, bool NT = false>
+template <typename T, int ROWS, bool KC, int BK>
 struct Stage {
     static constexpr int V = Vec16<T>::n;
     static constexpr int E = ROWS * BK / kThreads;
-    static constexpr int NC = E / V;  // 16-byte pieces per thread
-    static constexpr int NCR = KC ? NC : ROWS / (16 * V);  // RC: pieces per k-row and thread
+    static constexpr int NC = E / V;                              // 16-byte pieces per thread
+    static constexpr int TPK = BK / E;                            // KC: threads per row
+    static constexpr int TPR = ROWS / V < 16 ? ROWS / V : 16;     // RC: threads per k-row
+    static constexpr int NCR = KC ? NC : ROWS / (TPR * V);        // RC: pieces per k-row and thread
     static constexpr int PAD = 16 / sizeof(T);
     static constexpr int PITCH = KC ? (BK + PAD) : (ROWS + 4);
     static constexpr int ELEMS = KC ? ROWS * PITCH : BK * PITCH;
     static_assert(BK % 16 == 0 && E % V == 0 && (KC ? BK % E == 0 : (NC % NCR == 0 && NCR >= 1)), "stage split");
     typedef typename Vec16<T>::type vec_t;
+    typedef typename Mem16<T>::type mem_t;
 
     vec_t reg[NC];
 
     __device__ __forceinline__ static void place(int& row, int& k) {
         const int t = threadIdx.x;
         if (KC) {
-            row = t / (BK / E);
-            k = (t % (BK / E)) * E;
+            row = t / TPK;
+            k = (t % TPK) * (BK == 16 ? E : V);
         } else {
-            k = t / 16;
-            row = (t % 16) * V;
+            k = t / TPR;
+            row = (t % TPR) * V;
         }
     }
     // Offsets of piece c relative to piece 0: along the rows and along k.
-    __device__ __forceinline__ static constexpr int prow(int c) { return KC ? 0 : (c % NCR) * 16 * V; }
-    __device__ __forceinline__ static constexpr int pk(int c) { return KC ? c * V : (c / NCR) * 16; }
+    __device__ __forceinline__ static constexpr int prow(int c) { return KC ? 0 : (c % NCR) * TPR * V; }
+    __device__ __forceinline__ static constexpr int pk(int c) {
+        return KC ? (BK == 16 ? c * V : c * TPK * V) : (c / NCR) * (kThreads / TPR);
+    }
 
-    // FAST (interior stage: tile inside the matrix, 16-byte aligned):
-    // unconditional vector loads. Otherwise (edge tiles, the K tail, unaligned
-    // operands) piece by piece: a piece wholly inside is one vector load (VEC),
-    // one wholly outside is zero without a load, and only a piece straddling
-    // the edge is loaded element-wise from clamped addresses. Measured against
-    // element-wise loads for every piece (fp32, fp64 TFLOP/s): 2000 x 3000 x
-    // 2000 106.5 and 57.3 against 77.0 and 51.0; 4000^3 TN 123.4 and 58.4
-    // against 95.7 and 53.6; aligned shapes unchanged.
-    template <bool FAST>
-    __device__ __forceinline__ void load(const T* __restrict__ p, int64_t ld, int64_t row0, int64_t rows,
-                                         int64_t k0, int64_t kdim) {
+    // A stage whose BK k are all in range: unconditional vector loads.
+    // INSIDE: the tile's rows are too. Otherwise rows from `rows` up are
+    // clamped: a KC row past the end reads the last row again, an RC piece
+    // that would pass the end starts at rows - V instead (rows >= V) and
+    // store() moves its elements into place; what lands in rows past the end
+    // feeds only outputs that are never stored. Ragged matrices so run the
+    // same branch-free loop as whole tiles; guarded piece by piece
+    // and loaded element by element when unaligned, as before, the edge
+    // tiles set the time of the launch (fp32 1999 x 3001 x 1201 with
+    // alpha/beta and C, all odd: 150 us against 224).
+    template <bool INSIDE>
+    __device__ __forceinline__ void load(const T* __restrict__ p, int64_t ld, int64_t row0, int64_t rows, int64_t k0) {
         int r, k;
         place(r, k);
-        if (FAST) {
-            const T* src = KC ? p + (row0 + r) * ld + (k0 + k) : p + (k0 + k) * ld + (row0 + r);
+        if (INSIDE || KC) {
+            const int64_t row = INSIDE ? row0 + r : min(row0 + r, rows - 1);
+            const T* src = KC ? p + row * ld + (k0 + k) : p + (k0 + k) * ld + row;
 #pragma unroll
             for (int c = 0; c < NC; ++c) {
-                const vec_t* q = reinterpret_cast<const vec_t*>(KC ? src + pk(c) : src + pk(c) * ld + prow(c));
-                reg[c] = NT ? __builtin_nontemporal_load(q) : *q;
+                const mem_t* q = reinterpret_cast<const mem_t*>(KC ? src + pk(c) : src + pk(c) * ld + prow(c));
+                reg[c] = *q;
             }
         } else {
 #pragma unroll
             for (int c = 0; c < NC; ++c) {
-                const int64_t pr = row0 + r + prow(c);
-                const int64_t pkk = k0 + k + pk(c);
-                const bool inside = KC ? (pr < rows && pkk + V <= kdim) : (pkk < kdim && pr + V <= rows);
-                const bool outside = pr >= rows || pkk >= kdim;
-                if (VEC && inside) {
-                    reg[c] = *reinterpret_cast<const vec_t*>(KC ? p + pr * ld + pkk : p + pkk * ld + pr);
-                } else if (outside) {
+                const int64_t row = min(row0 + r + prow(c), rows - V);
+                const mem_t* q = reinterpret_cast<const mem_t*>(p + (k0 + k + pk(c)) * ld + row);
+                reg[c] = *q;
+            }
+        }
+    }
+
+    // The stage that passes K (zero from there), and every stage when an RC
+    // operand has fewer than V rows: a piece wholly inside is one vector
+    // load, one wholly outside is zero without a load, and only a piece
+    // straddling the edge is loaded element-wise from clamped addresses.
+    // Rows past `rows` are zero; store() must not move them.
+    __device__ __forceinline__ void load_tail(const T* __restrict__ p, int64_t ld, int64_t row0, int64_t rows,
+                                              int64_t k0, int64_t kdim) {
+        int r, k;
+        place(r, k);
 #pragma unroll
-                    for (int e = 0; e < V; ++e) reg[c][e] = T(0);
-                } else {
+        for (int c = 0; c < NC; ++c) {
+            const int64_t pr = row0 + r + prow(c);
+            const int64_t pkk = k0 + k + pk(c);
+            const bool inside = KC ? (pr < rows && pkk + V <= kdim) : (pkk < kdim && pr + V <= rows);
+            const bool outside = pr >= rows || pkk >= kdim;
+            if (inside) {
+                reg[c] = *reinterpret_cast<const mem_t*>(KC ? p + pr * ld + pkk : p + pkk * ld + pr);
+            } else if (outside) {
 #pragma unroll
-                    for (int e = 0; e < V; ++e) {
-                        const int64_t gr = pr + (KC ? 0 : e);
-                        const int64_t gk = pkk + (KC ? e : 0);
-                        const bool ok = gr < rows && gk < kdim;
-                        const T x = *(ok ? (KC ? p + gr * ld + gk : p + gk * ld + gr) : p);
-                        reg[c][e] = ok ? x : T(0);
-                    }
+                for (int e = 0; e < V; ++e) reg[c][e] = T(0);
+            } else {
+#pragma unroll
+                for (int e = 0; e < V; ++e) {
+                    const int64_t gr = pr + (KC ? 0 : e);
+                    const int64_t gk = pkk + (KC ? e : 0);
+                    const bool ok = gr < rows && gk < kdim;
+                    const T x = *(ok ? (KC ? p + gr * ld + gk : p + gk * ld + gr) : p);
+                    reg[c][e] = ok ? x : T(0);
                 }
             }
         }
@@ -116,6 +152,26 @@ struct Stage {
 #pragma unroll
         for (int c = 0; c < NC; ++c)
             *reinterpret_cast<vec_t*>(KC ? dst + pk(c) : dst + pk(c) * PITCH + prow(c)) = reg[c];
+    }
+
+    // After a clamped load<false> of an RC operand: each piece that was
+    // started early is moved down by its overshoot.
+    __device__ __forceinline__ void align(int64_t row0, int64_t rows) {
+        if (KC) return;
+        int r, k;
+        place(r, k);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            const int64_t over = row0 + r + prow(c) + V - rows;  // <= 0: not clamped; >= V: no row inside
+            const int s = over > 0 ? (int)over : 0;
+            vec_t x = reg[c];
+            if constexpr (V == 4) {
+                const vec_t y = (s & 2) ? vec_t{x[2], x[3], x[0], x[1]} : x;
+                reg[c] = (s & 1) ? vec_t{y[1], y[2], y[3], y[0]} : y;
+            } else {
+                reg[c] = (s & 1) ? vec_t{x[1], x[0]} : x;
+            }
+        }
     }
 
     // The four k values (MFMA steps 0..3 of 16-k pass kk) this lane feeds for
@@ -135,19 +191,14 @@ struct Stage {
     }
 };
 
-template <typename T, int BM, int BN, int FM, int FN, bool TA, bool TB, bool VEC, bool DOT, int NBUF, int BK,
-          bool PRIO>
+// FULL: M and N are multiples of the tile (no row or column clamping).
+template <typename T, int BM, int BN, int FM, int FN, bool TA, bool TB, bool FULL, bool DOT, int NBUF, int BK>
 __global__ __launch_bounds__(kThreads) void gemm_kernel(GemmArgs g) {
     typedef Mfma<T> MF;
     typedef typename MF::acc_t acc_t;
     // A rows are m: k-contiguous unless transposed. B rows are n: k-contiguous iff transposed.
-    typedef Stage<T, BM, !TA, VEC, BK> SA;
-    // The single-buffer small-M tile reads B once (one tile row; the launcher
-    // sends a batch-broadcast B elsewhere), so B's loads are non-temporal and
-    // leave the L2 to A, which every workgroup re-reads: AO->MO half
-    // transform 0.909-0.920 -> 0.899-0.900 ms, results bitwise equal.
-    // Non-temporal loads of A as well, or on tiles that re-read B, cost 7-18%.
-    typedef Stage<T, BN, TB, VEC, BK, NBUF == 1 && PRIO> SB;
+    typedef Stage<T, BM, !TA, BK> SA;
+    typedef Stage<T, BN, TB, BK> SB;
     // Each wavefront owns an (16 FM) x (16 FN) sub-tile: FM x FN MFMA blocks.
     constexpr int WM = 16 * FM, WN = 16 * FN;
     constexpr int WAVES_N = BN / WN;
@@ -193,15 +244,29 @@ __global__ __launch_bounds__(kThreads) void gemm_kernel(GemmArgs g) {
     SA sa;
     SB sb;
     const int64_t nk = (g.K + BK - 1) / BK;
-    // Stages 0 .. nfull-1 are interior for both operands.
-    const int64_t nfull = (VEC && m0 + BM <= g.M && n0 + BN <= g.N) ? g.K / BK : 0;
+    // Stages 0 .. nfull-1 have all their k in range (a row-contiguous operand
+    // with fewer rows than one vector takes the guarded loads throughout).
+    const int64_t nfull = (!TA || g.M >= Vec16<T>::n) && (TB || g.N >= Vec16<T>::n) ? g.K / BK : 0;
     // The lambdas below are always inlined: left as calls (which the inliner
     // chose for 64-deep stages), they capture acc by reference and the
     // accumulators go to scratch memory.
-    auto load = [&](int64_t k0, auto fast) __attribute__((always_inline)) {
-        constexpr bool F = decltype(fast)::value;
-        sa.template load<F>(A, g.lda, m0, g.M, k0, g.K);
-        sb.template load<F>(B, g.ldb, n0, g.N, k0, g.K);
+    auto load = [&](int64_t k0) __attribute__((always_inline)) {
+        sa.template load<FULL>(A, g.lda, m0, g.M, k0);
+        sb.template load<FULL>(B, g.ldb, n0, g.N, k0);
+    };
+    auto load_tail = [&](int64_t k0) __attribute__((always_inline)) {
+        sa.load_tail(A, g.lda, m0, g.M, k0, g.K);
+        sb.load_tail(B, g.ldb, n0, g.N, k0, g.K);
+    };
+    // Pieces that were clamped at the matrix edge (uniform: edge tiles only).
+    const bool edge_m = TA && !FULL && m0 + BM > g.M, edge_n = !TB && !FULL && n0 + BN > g.N;
+    auto store = [&](int b) __attribute__((always_inline)) {
+        sa.store(bufA(b));
+        sb.store(bufB(b));
+    };
+    auto align = [&]() __attribute__((always_inline)) {
+        if (edge_m) sa.align(m0, g.M);
+        if (edge_n) sb.align(n0, g.N);
     };
     auto compute = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
@@ -220,10 +285,13 @@ __global__ __launch_bounds__(kThreads) void gemm_kernel(GemmArgs g) {
         }
     };
     if (nk > 0) {
-        if (nfull > 0) load(0, std::true_type{});
-        else load(0, std::false_type{});
-        sa.store(bufA(0));
-        sb.store(bufB(0));
+        if (nfull > 0) {
+            load(0);
+            align();
+        } else {
+            load_tail(0);
+        }
+        store(0);
     }
     __syncthreads();
 
@@ -235,33 +303,22 @@ __global__ __launch_bounds__(kThreads) void gemm_kernel(GemmArgs g) {
     auto next = [&](int64_t kt) -> int { return NBUF == 2 ? (int)((kt & 1) ^ 1) : 0; };
     auto cur = [&](int64_t kt) -> int { return NBUF == 2 ? (int)(kt & 1) : 0; };
     int64_t kt = 0;
-    // PRIO (fp64): the wave issuing a stage's MFMAs runs at raised priority
-    // for the burst, so co-resident waves in their load/store phase do not
-    // delay the MFMA stream.
-    auto mfma_stage = [&](int b) __attribute__((always_inline)) {
-        if (PRIO && sizeof(T) == 8) __builtin_amdgcn_s_setprio(1);
-        compute(b);
-        if (PRIO && sizeof(T) == 8) __builtin_amdgcn_s_setprio(0);
-    };
     for (; kt + 1 < nfull; ++kt) {
-        load((kt + 1) * BK, std::true_type{});
-        mfma_stage(cur(kt));
+        load((kt + 1) * BK);
+        compute(cur(kt));
         __builtin_amdgcn_sched_barrier(0);
+        align();
         if (NBUF == 1) __syncthreads();
-        sa.store(bufA(next(kt)));
-        sb.store(bufB(next(kt)));
+        store(next(kt));
         __syncthreads();
     }
     for (; kt < nk; ++kt) {
         const bool more = kt + 1 < nk;
-        if (more) load((kt + 1) * BK, std::false_type{});
-        mfma_stage(cur(kt));
+        if (more) load_tail((kt + 1) * BK);
+        compute(cur(kt));
         __builtin_amdgcn_sched_barrier(0);
         if (NBUF == 1) __syncthreads();
-        if (more) {
-            sa.store(bufA(next(kt)));
-            sb.store(bufB(next(kt)));
-        }
+        if (more) store(next(kt));
         __syncthreads();
     }
 
@@ -273,66 +330,40 @@ __global__ __launch_bounds__(kThreads) void gemm_kernel(GemmArgs g) {
         const T* E1 = static_cast<const T*>(g.E1) + bat * g.e1s[4];
         const T* E2 = g.E2 ? static_cast<const T*>(g.E2) + bat * g.e2s[4] : nullptr;
         double sum = 0.0;
-        if constexpr (NBUF == 2) {
-            // Each 16x16 block's eight E loads (branch-free: rows and columns
-            // outside the matrix read element (0, 0)) go out together before
-            // its sums, which keep the order below. Loaded under the
-            // per-element bounds branches, every load waited out a full
-            // latency before its sum: 128 waits per lane at 128 x 128, and
-            // config 5's greedy path took 69.4 ms against 68.4 ms this way
-            // (results bitwise equal). The single-buffer small-M tile keeps
-            // the form below: the batches would cost it a wave per SIMD.
+        // Each 16x16 block's eight E loads (branch-free: rows and columns
+        // outside the matrix read element (0, 0)) go out together before
+        // its sums, which keep the order below. Loaded under the
+        // per-element bounds branches, every load waited out a full
+        // latency before its sum: 128 waits per lane at 128 x 128, and
+        // config 5's greedy path took 69.4 ms against 68.4 ms this way
+        // (results bitwise equal).
 #pragma unroll
-            for (int j = 0; j < FN; ++j) {
-                const int64_t col = n0 + wn0 + 16 * j + col_l;
-                const bool cok = col < g.N;
-                const uint32_t nh = fdiv((uint32_t)(cok ? col : 0), g.ndiv);
-                const uint32_t nl = (uint32_t)(cok ? col : 0) - nh * g.ndiv.d;
-                const int64_t o1n = nh * g.e1s[2] + nl * g.e1s[3];
-                const int64_t o2n = nh * g.e2s[2] + nl * g.e2s[3];
+        for (int j = 0; j < FN; ++j) {
+            const int64_t col = n0 + wn0 + 16 * j + col_l;
+            const bool cok = col < g.N;
+            const uint32_t nh = fdiv((uint32_t)(cok ? col : 0), g.ndiv);
+            const uint32_t nl = (uint32_t)(cok ? col : 0) - nh * g.ndiv.d;
+            const int64_t o1n = nh * g.e1s[2] + nl * g.e1s[3];
+            const int64_t o2n = nh * g.e2s[2] + nl * g.e2s[3];
 #pragma unroll
-                for (int i = 0; i < FM; ++i) {
-                    T e1v[4], e2v[4];
+            for (int i = 0; i < FM; ++i) {
+                T e1v[4], e2v[4];
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int64_t row = m0 + wm0 + 16 * i + MF::row(lgrp, r);
-                        const bool ok = cok && row < g.M;
-                        const uint32_t mh = fdiv((uint32_t)(ok ? row : 0), g.mdiv);
-                        const uint32_t ml = (uint32_t)(ok ? row : 0) - mh * g.mdiv.d;
-                        e1v[r] = E1[ok ? mh * g.e1s[0] + ml * g.e1s[1] + o1n : 0];
-                        if (E2) e2v[r] = E2[ok ? mh * g.e2s[0] + ml * g.e2s[1] + o2n : 0];
-                    }
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int64_t row = m0 + wm0 + 16 * i + MF::row(lgrp, r);
-                        if (cok && row < g.M) {
-                            T e = e1v[r];
-                            if (E2) e = e * e2v[r];
-                            sum += (double)(acc[i][j][r] * e);
-                        }
-                    }
+                for (int r = 0; r < 4; ++r) {
+                    const int64_t row = m0 + wm0 + 16 * i + MF::row(lgrp, r);
+                    const bool ok = cok && row < g.M;
+                    const uint32_t mh = fdiv((uint32_t)(ok ? row : 0), g.mdiv);
+                    const uint32_t ml = (uint32_t)(ok ? row : 0) - mh * g.mdiv.d;
+                    e1v[r] = E1[ok ? mh * g.e1s[0] + ml * g.e1s[1] + o1n : 0];
+                    if (E2) e2v[r] = E2[ok ? mh * g.e2s[0] + ml * g.e2s[1] + o2n : 0];
                 }
-            }
-        } else {
 #pragma unroll
-            for (int j = 0; j < FN; ++j) {
-                const int64_t col = n0 + wn0 + 16 * j + col_l;
-                const uint32_t nh = fdiv((uint32_t)col, g.ndiv);
-                const uint32_t nl = (uint32_t)col - nh * g.ndiv.d;
-                const int64_t o1n = nh * g.e1s[2] + nl * g.e1s[3];
-                const int64_t o2n = nh * g.e2s[2] + nl * g.e2s[3];
-#pragma unroll
-                for (int i = 0; i < FM; ++i) {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int64_t row = m0 + wm0 + 16 * i + MF::row(lgrp, r);
-                        if (row < g.M && col < g.N) {
-                            const uint32_t mh = fdiv((uint32_t)row, g.mdiv);
-                            const uint32_t ml = (uint32_t)row - mh * g.mdiv.d;
-                            T e = E1[mh * g.e1s[0] + ml * g.e1s[1] + o1n];
-                            if (E2) e = e * E2[mh * g.e2s[0] + ml * g.e2s[1] + o2n];
-                            sum += (double)(acc[i][j][r] * e);
-                        }
+                for (int r = 0; r < 4; ++r) {
+                    const int64_t row = m0 + wm0 + 16 * i + MF::row(lgrp, r);
+                    if (cok && row < g.M) {
+                        T e = e1v[r];
+                        if (E2) e = e * e2v[r];
+                        sum += (double)(acc[i][j][r] * e);
                     }
                 }
             }
@@ -387,12 +418,11 @@ __global__ __launch_bounds__(kThreads) void gemm_kernel(GemmArgs g) {
 
 // Store epilogue of the direct-B kernels: D = alpha * acc (+ beta * C) for
 // the 64 x BN tile at rows m0.., column tile tn of batch entry bat.
-// acc[a][b][r] is row m0 + 16 a + MF::row(lg, r), column col + b. When D's
-// (and C's) rows start 16-byte aligned (checked below), a lane's NB columns
-// are one 16-byte piece. The lane indices are formed again here rather than
-// held through the K loop.
-// PLAIN: no C, D's rows 16-byte aligned and the tile inside N (the caller
-// checked), so every row is one unconditional 16-byte store per lane.
+// acc[a][b][r] is row m0 + 16 a + MF::row(lg, r), column col + b; a lane's NB
+// columns are one 16-byte piece of D and of C. The lane indices are formed
+// again here rather than held through the K loop.
+// PLAIN: no C and the tile inside N (the caller checked), so every row is one
+// unconditional 16-byte store per lane.
 template <typename T, bool FULLM, bool PLAIN = false>
 __device__ __forceinline__ void directb_store(const GemmArgs& g, typename Mfma<T>::acc_t (&acc)[4][16 / sizeof(T)],
                                               int64_t bat, int64_t m0, int64_t tn) {
@@ -400,6 +430,7 @@ __device__ __forceinline__ void directb_store(const GemmArgs& g, typename Mfma<T
     constexpr int NB = 16 / sizeof(T);
     constexpr int BN = 64 * NB;
     typedef typename VecN<T, 16 / sizeof(T)>::type v16_t;
+    typedef typename Mem16<T>::type mem_t;
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));
     const int lg = (tid & 63) >> 4;
@@ -415,15 +446,13 @@ __device__ __forceinline__ void directb_store(const GemmArgs& g, typename Mfma<T
                 v16_t v;
 #pragma unroll
                 for (int b = 0; b < NB; ++b) v[b] = g.alpha != 1.0 ? alpha * acc[a][b][r] : acc[a][b][r];
-                *reinterpret_cast<v16_t*>(D + (m0 + 16 * a + MF::row(lg, r)) * g.ldd + col) = v;
+                *reinterpret_cast<mem_t*>(D + (m0 + 16 * a + MF::row(lg, r)) * g.ldd + col) = v;
             }
         return;
     }
     const T* C = g.C ? static_cast<const T*>(g.C) + bat * g.sC : nullptr;
-    const bool vecd = ((reinterpret_cast<uintptr_t>(D) | (uintptr_t)(g.ldd * sizeof(T))) & 15) == 0 &&
-                      (!C || ((reinterpret_cast<uintptr_t>(C) | (uintptr_t)(g.ldc * sizeof(T))) & 15) == 0);
-    const bool colok = col < g.N;  // N is a multiple of NB: all NB columns or none
-    if (C && vecd) {
+    const bool colok = col + NB <= g.N;  // all NB columns inside
+    if (C) {
         // A lane's NB columns of a row are one 16-byte piece of C and of D.
         // The C pieces of two row blocks (eight rows) go out together before
         // their stores: two memory round trips per tile instead of four, and
@@ -441,9 +470,7 @@ __device__ __forceinline__ void directb_store(const GemmArgs& g, typename Mfma<T
                 for (int r = 0; r < 4; ++r) {
                     const int64_t row = m0 + 16 * (a2 + h) + MF::row(lg, r);
                     const bool ok = (FULLM || row < g.M) && colok;
-                    const v16_t x = *reinterpret_cast<const v16_t*>(C + (ok ? row * g.ldc + col : 0));
-#pragma unroll
-                    for (int b = 0; b < NB; ++b) cv[h][r][b] = ok ? x[b] : T(0);
+                    cv[h][r] = *reinterpret_cast<const mem_t*>(C + (ok ? row * g.ldc + col : 0));
                 }
 #pragma unroll
             for (int h = 0; h < 2; ++h)
@@ -458,51 +485,47 @@ __device__ __forceinline__ void directb_store(const GemmArgs& g, typename Mfma<T
                         if (g.alpha != 1.0) v[b] = alpha * v[b];
                         v[b] = v[b] + beta * cv[h][r][b];
                     }
-                    *reinterpret_cast<v16_t*>(D + row * g.ldd + col) = v;
+                    *reinterpret_cast<mem_t*>(D + row * g.ldd + col) = v;
                 }
         }
-        return;
-    }
+    } else {
 #pragma unroll
-    for (int a = 0; a < 4; ++a) {
-        T cv[4][NB];
-        if (C) {
+        for (int a = 0; a < 4; ++a)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int64_t row = m0 + 16 * a + MF::row(lg, r);
-                const bool ok = (FULLM || row < g.M) && colok;
+                if ((!FULLM && row >= g.M) || !colok) continue;
+                v16_t v;
 #pragma unroll
-                for (int b = 0; b < NB; ++b) {
-                    const T x = C[ok ? row * g.ldc + col + b : 0];
-                    cv[r][b] = ok ? x : T(0);
+                for (int b = 0; b < NB; ++b) v[b] = g.alpha != 1.0 ? alpha * acc[a][b][r] : acc[a][b][r];
+                *reinterpret_cast<mem_t*>(D + row * g.ldd + col) = v;
+            }
+    }
+    if (g.N % NB) {
+        // The lane whose NB columns straddle N computed columns N - NB ..
+        // N - 1 (its B column was clamped): it stores those from col up.
+        if (col < g.N && !colok) {
+#pragma unroll
+            for (int a = 0; a < 4; ++a)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int64_t row = m0 + 16 * a + MF::row(lg, r);
+#pragma unroll
+                    for (int b = 1; b < NB; ++b) {
+                        const int64_t cb = g.N - NB + b;
+                        if (cb < col || (!FULLM && row >= g.M)) continue;
+                        T v = acc[a][b][r];
+                        if (g.alpha != 1.0) v = alpha * v;
+                        if (C) v = v + beta * C[row * g.ldc + cb];
+                        D[row * g.ldd + cb] = v;
+                    }
                 }
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int64_t row = m0 + 16 * a + MF::row(lg, r);
-            if ((!FULLM && row >= g.M) || !colok) continue;
-            v16_t v;
-#pragma unroll
-            for (int b = 0; b < NB; ++b) {
-                v[b] = acc[a][b][r];
-                if (g.alpha != 1.0) v[b] = alpha * v[b];
-                if (C) v[b] = v[b] + beta * cv[r][b];
-            }
-            T* d = D + row * g.ldd + col;
-            if (vecd) {
-                *reinterpret_cast<v16_t*>(d) = v;
-            } else {
-#pragma unroll
-                for (int b = 0; b < NB; ++b) d[b] = v[b];
-            }
         }
     }
 }
 
 // GEMM (or dot epilogue, DOT): fp64 on 64 x 128 tiles, fp32 on 64 x 256 tiles,
-// four waves each; N a multiple of NB (below), the last column tile may be
-// partial (not with DOT).
+// four waves each; N at least NB (below), the last column tile may be partial.
 // A (either layout) is staged through LDS one 64-row slab per workgroup,
 // double-buffered, one barrier per 16-k stage; rows from M up and k from K up
 // read as zero. B goes from memory straight into the MFMA operand registers:
@@ -527,7 +550,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     constexpr int BN = 64 * NB;         // tile columns: 128 (fp64), 256 (fp32)
     constexpr int SPL = TB ? 16 / sizeof(T) : 1;  // MFMA steps one B load feeds (TB: k-contiguous piece)
     typedef typename VecN<T, 16 / sizeof(T)>::type v16_t;
-    typedef Stage<T, 64, !TA, true, kBK> SA;  // A: a 64-row slab, [k][m] (TA) or [m][k] in LDS
+    typedef typename Mem16<T>::type mem_t;
+    typedef Stage<T, 64, !TA, kBK> SA;  // A: a 64-row slab, [k][m] (TA) or [m][k] in LDS
     __shared__ __attribute__((aligned(16))) T lds[2 * SA::ELEMS];
 
     // Tile order: the 64-row slabs of one column tile are adjacent (they
@@ -568,9 +592,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
         const int lg = lane >> 4;
         const int c = lane & 15;
         // The lane's first column, clamped into the matrix: in a last, partial
-        // column tile the lanes past N read column N - NB instead, and their
-        // results are never stored (a column of D depends on that column of B
-        // only).
+        // column tile the lanes that pass N read column N - NB instead; of
+        // their results only the columns a lane straddling N owns are stored
+        // (a column of D depends on that column of B only).
         const int64_t col0 = min(tn * BN + (threadIdx.x >> 6) * (16 * NB) + NB * c, g.N - NB);
         // B row-major: piece p (0..3) is k-row 16 t + 4 g + p, all NB columns.
         // B k-contiguous: piece p is column col0 + p % NB, k 16 t + 4 g +
@@ -583,7 +607,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
         SA sa;
         v16_t rb[4];  // B pieces of the current stage
         auto bload = [&](int64_t t, int p) __attribute__((always_inline)) {
-            const v16_t* q = reinterpret_cast<const v16_t*>(bptr(t, p));
+            const mem_t* q = reinterpret_cast<const mem_t*>(bptr(t, p));
             rb[p] = NT ? __builtin_nontemporal_load(q) : *q;
         };
         // Stage t's B where it may pass K: k from K up reads as zero.
@@ -597,9 +621,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                 rb[p][e] = ok ? x : T(0);
             }
         };
-        auto aload = [&](int64_t t) __attribute__((always_inline)) {
-            if (FULLM && t < nfull) sa.template load<true>(A, g.lda, m0, g.M, t * kBK, g.K);
-            else sa.template load<false>(A, g.lda, m0, g.M, t * kBK, g.K);
+        // A's stage t: interior, or (K % 16 left over) the last one.
+        auto aload = [&](int64_t t) __attribute__((always_inline)) { sa.template load<FULLM>(A, g.lda, m0, g.M, t * kBK); };
+        auto aload_tail = [&](int64_t t) __attribute__((always_inline)) { sa.load_tail(A, g.lda, m0, g.M, t * kBK, g.K); };
+        const bool edge_m = TA && !FULLM && m0 + 64 > g.M;  // clamped pieces (uniform)
+        auto astore = [&](int64_t t) __attribute__((always_inline)) {
+            if (edge_m && t < nfull) sa.align(m0, g.M);
+            sa.store(lds + (t & 1) * SA::ELEMS);
         };
         auto afrag = [&](const T* sbuf, int a, int s) __attribute__((always_inline)) -> T {
             return TA ? sbuf[(4 * lg + s) * SA::PITCH + 16 * a + c] : sbuf[(16 * a + c) * SA::PITCH + 4 * lg + s];
@@ -638,17 +666,16 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
         // 0.836 ms for the whole path, 12% fewer executed MFMA FLOP there.
         const int wave_u = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
         if (!DOT && tn * BN + (int64_t)wave_u * (16 * NB) >= g.N) {
-            aload(0);
-            sa.store(lds);
-            __syncthreads();
-            for (int64_t t = 0; t + 1 < nk; ++t) {
-                aload(t + 1);
-                sa.store(lds + ((t + 1) & 1) * SA::ELEMS);
+            for (int64_t t = 0; t < nk; ++t) {
+                if (t < nfull) aload(t);
+                else aload_tail(t);
+                astore(t);
                 __syncthreads();
             }
         } else {
-        aload(0);
-        sa.store(lds);
+        if (nfull > 0) aload(0);
+        else aload_tail(0);
+        astore(0);
         int64_t t = 0;
         // Only the vector loads of B lead into the main loop: with the
         // element-wise tail loads joining them there, the compiler's wait at
@@ -697,20 +724,20 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
-            sa.store(lds + ((t + 1) & 1) * SA::ELEMS);
+            astore(t + 1);
             __syncthreads();
         }
         }  // nfull > 0
         if (t + 1 < nk) {
             // The partial last stage (K not a multiple of 16).
-            aload(t + 1);
+            aload_tail(t + 1);
             const T* cur = lds + (t & 1) * SA::ELEMS;
 #pragma unroll
             for (int p = 0; p < 4; ++p) {
                 piece(cur, p);
                 bload_tail(t + 1, p);
             }
-            sa.store(lds + ((t + 1) & 1) * SA::ELEMS);
+            astore(t + 1);
             __syncthreads();
             ++t;
         }
@@ -746,7 +773,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                 // SIMD.
                 int lgb = lg;
                 asm volatile("" : "+v"(lgb));
-                const uint32_t cb = (uint32_t)(col + b);
+                // In a partial last column tile a lane that passes N computed
+                // columns N - NB .. N - 1; it owns those from col up.
+                const int64_t cw = min(col, g.N - NB) + b;
+                const bool cok = cw >= col;
+                const uint32_t cb = (uint32_t)(cok ? cw : 0);
                 const uint32_t nh = fdiv(cb, g.ndiv);
                 const uint32_t nl = cb - nh * g.ndiv.d;
                 const int64_t o1n = nh * g.e1s[2] + nl * g.e1s[3];
@@ -757,7 +788,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         const int64_t row = m0 + 16 * a + MF::row(lgb, r);
-                        const bool ok = FULLM || row < g.M;
+                        const bool ok = (FULLM || row < g.M) && cok;
                         const uint32_t rr = (uint32_t)(ok ? row : 0);
                         const uint32_t mh = fdiv(rr, g.mdiv);
                         const uint32_t ml = rr - mh * g.mdiv.d;
@@ -767,7 +798,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         const int64_t row = m0 + 16 * a + MF::row(lgb, r);
-                        if (FULLM || row < g.M) {
+                        if ((FULLM || row < g.M) && cok) {
                             T e = e1v[r];
                             if (HE2) e = e * e2v[r];
                             sum += (double)(acc[a][b][r] * e);
@@ -788,8 +819,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     }
 }
 
-// Persistent form of gemm_directb_kernel (store epilogue, no C, D 16-byte
-// aligned, whole 64-row and BN-column tiles, K a positive multiple of 16): each workgroup walks a list of tiles
+// Persistent form of gemm_directb_kernel (store epilogue, no C, whole 64-row and BN-column tiles, K a positive multiple of 16): each workgroup walks a list of tiles
 // and the stages of consecutive tiles form one software pipeline. The next
 // tile's first stage (A slab into LDS, B pieces into registers) is loaded
 // during the current tile's last MFMAs, and the current tile's stores are
@@ -807,7 +837,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     constexpr int BN = 64 * NB;
     constexpr int SPL = TB ? 16 / sizeof(T) : 1;
     typedef typename VecN<T, 16 / sizeof(T)>::type v16_t;
-    typedef Stage<T, 64, !TA, true, kBK> SA;
+    typedef typename Mem16<T>::type mem_t;
+    typedef Stage<T, 64, !TA, kBK> SA;
     __shared__ __attribute__((aligned(16))) T lds[2 * SA::ELEMS];
 
     const int64_t tiles = g.tiles_m * g.tiles_n;
@@ -845,7 +876,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     v16_t rb[4];
     auto bload = [&](const T* B, int64_t t, int p) __attribute__((always_inline)) {
         const T* q = (TB ? B + (int64_t)(p % NB) * g.ldb + 16 * t + SPL * (p / NB) : B + (16 * t + p) * g.ldb) + boff;
-        rb[p] = NT ? __builtin_nontemporal_load(reinterpret_cast<const v16_t*>(q)) : *reinterpret_cast<const v16_t*>(q);
+        rb[p] = NT ? __builtin_nontemporal_load(reinterpret_cast<const mem_t*>(q)) : *reinterpret_cast<const mem_t*>(q);
     };
     auto afrag = [&](const T* sbuf, int a, int s) __attribute__((always_inline)) -> T {
         return TA ? sbuf[(4 * lg + s) * SA::PITCH + 16 * a + c] : sbuf[(16 * a + c) * SA::PITCH + 4 * lg + s];
@@ -876,7 +907,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     };
 
     Tile cur = tile(id);
-    sa.template load<true>(cur.A, g.lda, cur.m0, g.M, 0, g.K);
+    sa.template load<true>(cur.A, g.lda, cur.m0, g.M, 0);
     sa.store(lds);
 #pragma unroll
     for (int p = 0; p < 4; ++p) bload(cur.B, 0, p);
@@ -888,7 +919,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
 #pragma unroll
             for (int b = 0; b < NB; ++b) acc[a][b] = acc_t{0, 0, 0, 0};
         for (int64_t t = 0; t + 1 < nk; ++t) {
-            sa.template load<true>(cur.A, g.lda, cur.m0, g.M, (t + 1) * kBK, g.K);
+            sa.template load<true>(cur.A, g.lda, cur.m0, g.M, (t + 1) * kBK);
             const T* sb = lds + buf * SA::ELEMS;
 #pragma unroll
             for (int p = 0; p < 4; ++p) {
@@ -904,7 +935,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
         const int64_t nid = id + per;
         const bool more = nid < hi;
         const Tile nxt = tile(more ? nid : id);
-        if (more) sa.template load<true>(nxt.A, g.lda, nxt.m0, g.M, 0, g.K);
+        if (more) sa.template load<true>(nxt.A, g.lda, nxt.m0, g.M, 0);
         const T* sb = lds + buf * SA::ELEMS;
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
@@ -951,7 +982,8 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_directb_stream_kernel(GemmAr
     constexpr int NB = 4;
     constexpr int BN = 64 * NB;
     typedef typename Vec16<double>::type v16_t;
-    typedef Stage<double, 64, false, true, kBK> SA;
+    typedef Mem16<double>::type mem_t;
+    typedef Stage<double, 64, false, kBK> SA;
     __shared__ __attribute__((aligned(16))) double lds[2 * SA::ELEMS];
 
     // Hardware workgroup w runs on XCD w % 8; the tiles are split into eight
@@ -991,7 +1023,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_directb_stream_kernel(GemmAr
         const double* q = B + (16 * t + p) * g.ldb + boff;
 #pragma unroll
         for (int j = 0; j < NB / 2; ++j) {
-            const v16_t* qq = reinterpret_cast<const v16_t*>(q + 32 * j);
+            const mem_t* qq = reinterpret_cast<const mem_t*>(q + 32 * j);
             rb[p][j] = NT ? __builtin_nontemporal_load(qq) : *qq;
         }
     };
@@ -1020,7 +1052,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_directb_stream_kernel(GemmAr
     // One stage of the current tile from LDS buffer buf; stage tn1 of tile
     // nxt is loaded behind it when `more`.
     auto stage = [&](int buf, bool more, const Tile& nxt, int64_t tn1) __attribute__((always_inline)) {
-        if (more) sa.template load<true>(nxt.A, g.lda, nxt.m0, g.M, tn1 * kBK, g.K);
+        if (more) sa.template load<true>(nxt.A, g.lda, nxt.m0, g.M, tn1 * kBK);
         const double* sb = lds + buf * SA::ELEMS;
 #pragma unroll
         for (int p = 0; p < 3; ++p) {
@@ -1058,13 +1090,13 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_directb_stream_kernel(GemmAr
                     v[0] = acc[a][2 * j][r];
                     v[1] = acc[a][2 * j + 1][r];
                     if (alpha != 1.0) v = v * alpha;
-                    __builtin_nontemporal_store(v, reinterpret_cast<v16_t*>(D + row * g.ldd + col + 32 * j));
+                    __builtin_nontemporal_store(v, reinterpret_cast<mem_t*>(D + row * g.ldd + col + 32 * j));
                 }
             }
     };
 
     Tile cur = tile(id);
-    sa.template load<true>(cur.A, g.lda, cur.m0, g.M, 0, g.K);
+    sa.template load<true>(cur.A, g.lda, cur.m0, g.M, 0);
     sa.store(lds);
 #pragma unroll
     for (int p = 0; p < 4; ++p) bload(cur.B, 0, p);
@@ -1122,14 +1154,12 @@ static int launch_directb(GemmArgs& g, bool ta, bool tb, bool nt, hipStream_t st
     // rounds (4096^3, 64 x 512^3 without C) it measured 1-2% slower, and its
     // other layouts spill registers.
     const int64_t slots = (int64_t)device_cus() / kNumXcd * 4;
-    const bool vecd = ((reinterpret_cast<uintptr_t>(g.D) | (uintptr_t)(g.ldd * sizeof(T)) |
-                        (uintptr_t)(g.sD * sizeof(T))) & 15) == 0;
     // fp64 with at most two row tiles and at least three 64 x 256 tiles per
     // workgroup at two per CU: the streaming kernel.
     if constexpr (sizeof(T) == 8 && !DOT) {
         const int64_t stiles = g.tiles_m * (g.N / 256) * g.batch;
         const int64_t sgrid = (int64_t)device_cus() / kNumXcd * kNumXcd * 2;
-        if (ta && !tb && full && !g.C && vecd && g.N % 256 == 0 && g.K >= kBK && g.K % kBK == 0 &&
+        if (ta && !tb && full && !g.C && g.N % 256 == 0 && g.K >= kBK && g.K % kBK == 0 &&
             g.tiles_m <= 2 && stiles >= 3 * sgrid) {
             g.tiles_n = g.N / 256;
             const dim3 grid((unsigned)sgrid), block(kThreads);
@@ -1138,7 +1168,7 @@ static int launch_directb(GemmArgs& g, bool ta, bool tb, bool nt, hipStream_t st
             return check_launch("tt_gemm");
         }
     }
-    if (!DOT && ta && !tb && full && !g.C && vecd && g.N % BN == 0 && g.K >= kBK && g.K % kBK == 0 &&
+    if (!DOT && ta && !tb && full && !g.C && g.N % BN == 0 && g.K >= kBK && g.K % kBK == 0 &&
         total >= 3 * slots * kNumXcd) {
         const dim3 grid((unsigned)(slots * kNumXcd)), block(kThreads);
         if (nt) hipLaunchKernelGGL((gemm_directb_persistent_kernel<T, true, false, true>), grid, block, 0, st, g);
@@ -1161,15 +1191,16 @@ static int launch_directb(GemmArgs& g, bool ta, bool tb, bool nt, hipStream_t st
     return check_launch("tt_gemm");
 }
 
-template <typename T, int BM, int BN, int FM, int FN, bool DOT, int NBUF = 2, int BK = kBK, bool PRIO = false>
-static int launch_tile(GemmArgs& g, bool ta, bool tb, bool vec, hipStream_t st) {
+template <typename T, int BM, int BN, int FM, int FN, bool DOT, int NBUF = 2, int BK = kBK>
+static int launch_tile(GemmArgs& g, bool ta, bool tb, hipStream_t st) {
     g.tiles_m = (g.M + BM - 1) / BM;
     g.tiles_n = (g.N + BN - 1) / BN;
     const int64_t total = g.tiles_m * g.tiles_n * g.batch;
     if (total > 0x7fffffffLL) return set_error(TT_UNSUPPORTED, "tt_gemm: %lld tiles exceed one launch", (long long)total);
+    const bool full = g.M % BM == 0 && g.N % BN == 0;
     dim3 grid((unsigned)total), block(kThreads);
-#define TT_GEMM_CASE(TA, TB, VC) \
-    if (ta == TA && tb == TB && vec == VC) hipLaunchKernelGGL((gemm_kernel<T, BM, BN, FM, FN, TA, TB, VC, DOT, NBUF, BK, PRIO>), grid, block, 0, st, g);
+#define TT_GEMM_CASE(TA, TB, F) \
+    if (ta == TA && tb == TB && full == F) hipLaunchKernelGGL((gemm_kernel<T, BM, BN, FM, FN, TA, TB, F, DOT, NBUF, BK>), grid, block, 0, st, g);
     TT_GEMM_CASE(false, false, false)
     TT_GEMM_CASE(false, false, true)
     TT_GEMM_CASE(false, true, false)
@@ -1188,113 +1219,87 @@ static int launch_tile(GemmArgs& g, bool ta, bool tb, bool vec, hipStream_t st) 
 // transposed), the layouts whose 32-row stage the staging supports. The k
 // order per output is the other tiles' (16-deep passes in order).
 template <typename T, int BK>
-static int launch_small(GemmArgs& g, bool vec, hipStream_t st) {
+static int launch_small(GemmArgs& g, hipStream_t st) {
     g.tiles_m = (g.M + 31) / 32;
     g.tiles_n = (g.N + 31) / 32;
     const int64_t total = g.tiles_m * g.tiles_n * g.batch;
     if (total > 0x7fffffffLL) return set_error(TT_UNSUPPORTED, "tt_gemm: %lld tiles exceed one launch", (long long)total);
     const dim3 grid((unsigned)total), block(kThreads);
-    if (vec) hipLaunchKernelGGL((gemm_kernel<T, 32, 32, 1, 1, false, true, true, false, 1, BK, false>), grid, block, 0, st, g);
-    else hipLaunchKernelGGL((gemm_kernel<T, 32, 32, 1, 1, false, true, false, false, 1, BK, false>), grid, block, 0, st, g);
+    hipLaunchKernelGGL((gemm_kernel<T, 32, 32, 1, 1, false, true, false, false, 1, BK>), grid, block, 0, st, g);
     return check_launch("tt_gemm");
 }
 
 template <typename T, bool DOT>
 static int gemm_typed(GemmArgs& g, bool ta, bool tb, hipStream_t st) {
     constexpr int V = Vec16<T>::n;
-    auto ok16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-    // 16-byte vectors need aligned bases, leading dimensions and batch strides.
-    bool vec = ok16(g.A) && ok16(g.B) && g.lda % V == 0 && g.ldb % V == 0;
-    if (g.batch > 1) vec = vec && g.sA % V == 0 && g.sB % V == 0;
     // One 32 x 32 tile per batch entry and K within one deep stage (the
     // DF-MP2 pair block 'ap,bp->ab' of config 1: 32 x 32 x 96).
     constexpr int64_t KS = 512 / sizeof(T);  // 128 fp32, 64 fp64
     if (!DOT && !ta && tb && g.M <= 32 && g.N <= 32 && g.K <= KS) {
-        if (g.K <= KS / 2) return launch_small<T, KS / 2>(g, vec, st);
-        return launch_small<T, KS>(g, vec, st);
+        if (g.K <= KS / 2) return launch_small<T, KS / 2>(g, st);
+        return launch_small<T, KS>(g, st);
     }
-    // Small-M (e.g. the AO->MO half transform, M = nocc): 64 x 128 tiles of
-    // four 32 x 64 wavefront tiles keep registers and LDS low enough for
-    // several workgroups per CU, i.e. more loads in flight on a long stream.
-    // Batched short-K fp64 (e.g. 64 x 512^3): three 64 x 128 workgroups per
-    // CU instead of two 128 x 128 ones overlap one workgroup's prologue and
-    // epilogue with the others' MFMAs (measured 62% -> 70% of fp64 peak;
-    // unbatched and fp32 cases measured no gain).
-    // fp64 small-M (the AO->MO half transform: M = nocc, K = nbasis, N =
-    // nbasis * naux): one LDS stage buffer (26 KB) gives four workgroups per
-    // CU instead of three, and the wave issuing a stage's MFMAs raises its
-    // priority for the burst. Same box, results bitwise equal: 64 x 786432 x
-    // 512 0.928-0.952 -> 0.895-0.927 ms (+2-3%). Raised priority measured
-    // slower for the batched and large fp64 tiles (64 x 512^3: +12% time), so
-    // it stays on this tile only. This tile streams B (non-temporal loads), so
-    // a B broadcast over the batch (stride 0, re-read per batch entry) takes
-    // the two-buffer tile below.
     // fp64: A through LDS, B straight into the MFMA registers
-    // (gemm_directb_kernel above), non-temporal when B is read once (M <= 64).
-    // With B row-major and N a multiple of 128, same box, alternating,
-    // bitwise equal, against the LDS-staged tiles below: 4096^3 with alpha/beta 1.952 against 2.082
-    // ms (NN 1.944 against 2.069, TN 1.965 against 2.171), 4096^2 x 512 0.258
-    // against 0.274 ms, 64 x 512^3 with alpha/beta and C 0.275 against 0.292
-    // ms, the AO->MO transform's two GEMMs 0.885 against 0.914 and 0.492
-    // against 0.520 ms. With N % 128 columns left over, a second launch for
-    // them ran alone after the first (nocc 50, N = 100002: 0.198 against
-    // 0.146 ms); a partial last tile in the same launch (below) takes 0.144.
-    // B k-contiguous (NT, TT) takes the same kernel, and so does the dot
-    // epilogue when M is a multiple of 64 (with row masking its epilogue
-    // spills). Same box, alternating: 4096^3 NT 2.026 against 2.130 ms and TT
-    // 2.025 against 2.104 ms (bitwise equal); the fused contraction of config
-    // 5 (dot GEMM 160000 x 16384 x 800, B k-contiguous) 66.2-66.4 against
-    // 67.9-68.0 ms, the sum equal to 2e-15 (another order of the per-tile
-    // sums).
-    // Any even N (a last, partial column tile clamps its columns; the dot
-    // epilogue keeps N a multiple of 128, any M: rows past M read A as zero
-    // and are left out of the sum). Same box, alternating, bitwise
-    // equal, against the LDS-staged tiles: 3000 x 3000 x 1000 with alpha/beta
-    // 0.331 against 0.438 ms, NT 0.382 against 0.426 ms, 8192 x 200 x 2048
-    // 0.145 against 0.186 ms, config 5's optimal-order GEMM (400 x 128 x 800
-    // x 400) 0.580 against 0.629 ms. The fp32 tile lost on such shapes (3000
-    // x 3000 x 1000 0.221 against 0.212 ms), so fp32 keeps whole tiles.
-    if constexpr (sizeof(T) == 8)
-        if (vec && (DOT ? g.N % 128 == 0 : g.N % 2 == 0))
+    // (gemm_directb_kernel above), non-temporal when B is read once (M <= 64
+    // and B not broadcast over the batch). Same box, alternating, bitwise
+    // equal, against LDS-staged tiles: 4096^3 with alpha/beta 1.952 against
+    // 2.082 ms (NN 1.944 against 2.069, TN 1.965 against 2.171, NT 2.026
+    // against 2.130, TT 2.025 against 2.104), 4096^2 x 512 0.258 against
+    // 0.274 ms, 64 x 512^3 with alpha/beta and C 0.275 against 0.292 ms, the
+    // AO->MO transform's two GEMMs 0.885 against 0.914 and 0.492 against
+    // 0.520 ms; partial column tiles (3000 x 3000 x 1000 with alpha/beta 0.331
+    // against 0.438 ms, NT 0.382 against 0.426, 8192 x 200 x 2048 0.145 against
+    // 0.186 ms). Odd N, leading dimensions and batch strides take it too
+    // (2999 x 3001 x 1001 with alpha/beta 306 against 713 us on guarded,
+    // element-wise LDS tiles, aligned 3000 x 3000 x 1000 311 us; 21 x 150 x
+    // 150 x 555 NT 42 against 112 us). With the dot epilogue: config 5's GEMM
+    // (160000 x 16384 x 800, B k-contiguous) 66.2-66.4 against 67.9-68.0 ms,
+    // 16900 x 900 x 450 (both extents ragged) 0.31 against 0.35 ms, the sum
+    // equal to 2e-15 (another order of the per-tile sums).
+    // What is left for fp64 (N = 1, or a transposed A of one row: no whole
+    // 16-byte piece along a row-contiguous operand) runs on the LDS tiles.
+    if constexpr (sizeof(T) == 8) {
+        if (g.N >= V && (!ta || g.M >= V))
             return launch_directb<T, DOT>(g, ta, tb, g.M <= 64 && (g.batch == 1 || g.sB != 0), st);
-    // fp32 on 64 x 256 tiles (four 16-column MFMA blocks per wave, so a lane's
-    // B piece is still 16 bytes): within 1-2% of the LDS-staged tiles, ahead
-    // on short K (same box, alternating, bitwise equal: 4096^2 x 512 0.1345
-    // against 0.1364 ms, 64 x 512^3 with alpha/beta and C 0.1397 against
-    // 0.1414 ms, 4096^3 0.988 against 0.990 ms).
-    // fp32, both operands not transposed, whole 256 x 256 tiles in whole
-    // rounds of one tile per CU (at least 95% of the last round busy), without
-    // C or with K >= 1024: the 256 x 256 LDS tile (tt_gemm_big.hip), bitwise
-    // equal to the tiles below. Same box, alternating, fraction of the fp32
-    // peak against the 64 x 256 direct-B tile: 4096^3 with alpha/beta and C
-    // 0.93 against 0.88; 64 x 512^3 without C 0.834 against 0.806, 16 x
-    // 1024^3 with C 0.866 against 0.845. A partial last round loses (6144^2 x
-    // 2048, 2.25 rounds: 1.444 against 1.118 ms), and so does a short K with
-    // C, whose epilogue one wave per SIMD cannot hide (64 x 512^3 with C
-    // 0.785 against 0.801, 128 x 512^3 with C 0.760 against 0.799).
-    if constexpr (sizeof(T) == 4 && !DOT)
-        if (gemm_big_f32_fits(ta, tb, g) && (!g.C || g.K >= 1024)) {
-            const int64_t tiles = (g.M / 256) * (g.N / 256) * g.batch, cus = device_cus();
-            const int64_t rounds = (tiles + cus - 1) / cus;
-            if (tiles >= cus && 100 * tiles >= 95 * rounds * cus) return gemm_big_f32_launch(g, st);
+        if (g.M > 64) return launch_tile<T, 256, 64, 4, 4, DOT>(g, ta, tb, st);
+        return launch_tile<T, 64, 128, 2, 4, DOT>(g, ta, tb, st);
+    } else {
+        // fp32 direct-B on 64 x 256 tiles (four 16-column MFMA blocks per wave, so
+        // a lane's B piece is still 16 bytes): within 1-2% of the LDS-staged
+        // tiles, ahead on short K (same box, alternating, bitwise equal: 4096^2 x
+        // 512 0.1345 against 0.1364 ms, 64 x 512^3 with alpha/beta and C 0.1397
+        // against 0.1414 ms, 4096^3 0.988 against 0.990 ms). Whole column tiles
+        // only: 3000 x 3000 x 1000 0.221 against 0.212 ms.
+        // fp32, both operands not transposed, whole 256 x 256 tiles in whole
+        // rounds of one tile per CU (at least 95% of the last round busy), without
+        // C or with K >= 1024: the 256 x 256 LDS tile (tt_gemm_big.hip), bitwise
+        // equal to the tiles below. Same box, alternating, fraction of the fp32
+        // peak against the 64 x 256 direct-B tile: 4096^3 with alpha/beta and C
+        // 0.93 against 0.88; 64 x 512^3 without C 0.834 against 0.806, 16 x
+        // 1024^3 with C 0.866 against 0.845. A partial last round loses (6144^2 x
+        // 2048, 2.25 rounds: 1.444 against 1.118 ms), and so does a short K with
+        // C, whose epilogue one wave per SIMD cannot hide (64 x 512^3 with C
+        // 0.785 against 0.801, 128 x 512^3 with C 0.760 against 0.799).
+        if constexpr (!DOT) {
+            if (gemm_big_f32_fits(ta, tb, g) && (!g.C || g.K >= 1024)) {
+                const int64_t tiles = (g.M / 256) * (g.N / 256) * g.batch, cus = device_cus();
+                const int64_t rounds = (tiles + cus - 1) / cus;
+                if (tiles >= cus && 100 * tiles >= 95 * rounds * cus) return gemm_big_f32_launch(g, st);
+            }
+            if (!tb && g.N % 256 == 0 && (!ta || g.M >= V))
+                return launch_directb<T, DOT>(g, ta, false, g.M <= 64 && (g.batch == 1 || g.sB != 0), st);
         }
-    if constexpr (sizeof(T) == 4 && !DOT)
-        if (!tb && vec && g.N % 256 == 0)
-            return launch_directb<T, DOT>(g, ta, false, g.M <= 64 && (g.batch == 1 || g.sB != 0), st);
-    if (sizeof(T) == 8 && !DOT && g.M <= 64 && (g.batch == 1 || g.sB != 0))
-        return launch_tile<T, 64, 128, 2, 4, DOT, 1, kBK, true>(g, ta, tb, vec, st);
-    if (g.M <= 64 || (sizeof(T) == 8 && g.batch > 1 && g.K <= 1024))
-        return launch_tile<T, 64, 128, 2, 4, DOT>(g, ta, tb, vec, st);
-    if (g.N <= 64) return launch_tile<T, 256, 64, 4, 4, DOT>(g, ta, tb, vec, st);
-    // Small grids: fewer than 448 128 x 128 tiles leave CUs idle; 64 x 128
-    // tiles double the grid (fp32, fp64 TFLOP/s against 128 x 128: 1024^3 41.9
-    // and 25.9 against 21.9 and 14.6; 2000 x 3000 x 2000 77.2 and 50.9 against
-    // 59.5 and 39.4; 2048^3 112.4 and 60.3 against 90.8 and 59.8; at 484 tiles,
-    // 2816^3, 120.4 and 60.7 against 131.3 and 62.0). Results are identical
-    // (the k order per output does not depend on the tile).
-    if (((g.M + 127) / 128) * ((g.N + 127) / 128) * g.batch < 448)
-        return launch_tile<T, 64, 128, 2, 4, DOT>(g, ta, tb, vec, st);
-    return launch_tile<T, 128, 128, 4, 4, DOT>(g, ta, tb, vec, st);
+        if (g.M <= 64) return launch_tile<T, 64, 128, 2, 4, DOT>(g, ta, tb, st);
+        if (g.N <= 64) return launch_tile<T, 256, 64, 4, 4, DOT>(g, ta, tb, st);
+        // Small grids: fewer than 448 128 x 128 tiles leave CUs idle; 64 x 128
+        // tiles double the grid (TFLOP/s against 128 x 128: 1024^3 41.9 against
+        // 21.9; 2000 x 3000 x 2000 77.2 against 59.5; 2048^3 112.4 against
+        // 90.8; at 484 tiles, 2816^3, 120.4 against 131.3). Results are
+        // identical (the k order per output does not depend on the tile).
+        if (((g.M + 127) / 128) * ((g.N + 127) / 128) * g.batch < 448)
+            return launch_tile<T, 64, 128, 2, 4, DOT>(g, ta, tb, st);
+        return launch_tile<T, 128, 128, 4, 4, DOT>(g, ta, tb, st);
+    }
 }
 
 int gemm_dispatch(int dtype, bool ta, bool tb, GemmArgs& g, hipStream_t st) {
