@@ -19,177 +19,9 @@
 #include <type_traits>
 
 #include "tt_gemm.hpp"
+#include "tt_stage.hpp"
 
 namespace tt {
-
-constexpr int kBK = 16;
-constexpr int kThreads = 256;
-
-
-// 16 bytes of T in memory at T's own alignment. gfx950 serves a 16-byte global
-// access at any element address, so operands, leading dimensions and batch
-// strides of any parity take the vector loads and stores; an access that is
-// not 16-byte aligned only touches one cache line more now and then.
-template <typename T>
-struct Mem16 {
-    typedef T type __attribute__((ext_vector_type(16 / sizeof(T)), aligned(sizeof(T))));
-};
-
-// One operand's ROWS x BK stage: global -> registers -> LDS, plus fragment reads.
-// KC: element (row, k) at p[row * ld + k]; otherwise at p[k * ld + row].
-// Each thread stages E = ROWS * BK / 256 elements as NC 16-byte pieces:
-//   KC: row t / TPK; BK = 16: one contiguous chunk from k = (t % TPK) E; deeper
-//       stages: pieces (t % TPK) + TPK c, so an instruction's lanes read
-//       TPK * 16 contiguous bytes of each row;
-//   RC: TPR threads per k-row, k-rows t / TPR + (256 / TPR) j; within a k-row a
-//       thread's pieces are (t % TPR) + TPR c, so every instruction covers
-//       TPR * 16 contiguous bytes of the k-row (coalesced loads,
-//       conflict-free stores).
-// RC k-rows are padded by 4 elements: the four lane groups of a fragment read
-// (k-rows 4 g + s) then land on disjoint LDS banks.
-template <typename T, int ROWS, bool KC, int BK>
-struct Stage {
-    static constexpr int V = Vec16<T>::n;
-    static constexpr int E = ROWS * BK / kThreads;
-    static constexpr int NC = E / V;                              // 16-byte pieces per thread
-    static constexpr int TPK = BK / E;                            // KC: threads per row
-    static constexpr int TPR = ROWS / V < 16 ? ROWS / V : 16;     // RC: threads per k-row
-    static constexpr int NCR = KC ? NC : ROWS / (TPR * V);        // RC: pieces per k-row and thread
-    static constexpr int PAD = 16 / sizeof(T);
-    static constexpr int PITCH = KC ? (BK + PAD) : (ROWS + 4);
-    static constexpr int ELEMS = KC ? ROWS * PITCH : BK * PITCH;
-    static_assert(BK % 16 == 0 && E % V == 0 && (KC ? BK % E == 0 : (NC % NCR == 0 && NCR >= 1)), "stage split");
-    typedef typename Vec16<T>::type vec_t;
-    typedef typename Mem16<T>::type mem_t;
-
-    vec_t reg[NC];
-
-    __device__ __forceinline__ static void place(int& row, int& k) {
-        const int t = threadIdx.x;
-        if (KC) {
-            row = t / TPK;
-            k = (t % TPK) * (BK == 16 ? E : V);
-        } else {
-            k = t / TPR;
-            row = (t % TPR) * V;
-        }
-    }
-    // Offsets of piece c relative to piece 0: along the rows and along k.
-    __device__ __forceinline__ static constexpr int prow(int c) { return KC ? 0 : (c % NCR) * TPR * V; }
-    __device__ __forceinline__ static constexpr int pk(int c) {
-        return KC ? (BK == 16 ? c * V : c * TPK * V) : (c / NCR) * (kThreads / TPR);
-    }
-
-    // A stage whose BK k are all in range: unconditional vector loads.
-    // INSIDE: the tile's rows are too. Otherwise rows from `rows` up are
-    // clamped: a KC row past the end reads the last row again, an RC piece
-    // that would pass the end starts at rows - V instead (rows >= V) and
-    // store() moves its elements into place; what lands in rows past the end
-    // feeds only outputs that are never stored. Ragged matrices so run the
-    // same branch-free loop as whole tiles; guarded piece by piece
-    // and loaded element by element when unaligned, as before, the edge
-    // tiles set the time of the launch (fp32 1999 x 3001 x 1201 with
-    // alpha/beta and C, all odd: 150 us against 224).
-    template <bool INSIDE>
-    __device__ __forceinline__ void load(const T* __restrict__ p, int64_t ld, int64_t row0, int64_t rows, int64_t k0) {
-        int r, k;
-        place(r, k);
-        if (INSIDE || KC) {
-            const int64_t row = INSIDE ? row0 + r : min(row0 + r, rows - 1);
-            const T* src = KC ? p + row * ld + (k0 + k) : p + (k0 + k) * ld + row;
-#pragma unroll
-            for (int c = 0; c < NC; ++c) {
-                const mem_t* q = reinterpret_cast<const mem_t*>(KC ? src + pk(c) : src + pk(c) * ld + prow(c));
-                reg[c] = *q;
-            }
-        } else {
-#pragma unroll
-            for (int c = 0; c < NC; ++c) {
-                const int64_t row = min(row0 + r + prow(c), rows - V);
-                const mem_t* q = reinterpret_cast<const mem_t*>(p + (k0 + k + pk(c)) * ld + row);
-                reg[c] = *q;
-            }
-        }
-    }
-
-    // The stage that passes K (zero from there), and every stage when an RC
-    // operand has fewer than V rows: a piece wholly inside is one vector
-    // load, one wholly outside is zero without a load, and only a piece
-    // straddling the edge is loaded element-wise from clamped addresses.
-    // Rows past `rows` are zero; store() must not move them.
-    __device__ __forceinline__ void load_tail(const T* __restrict__ p, int64_t ld, int64_t row0, int64_t rows,
-                                              int64_t k0, int64_t kdim) {
-        int r, k;
-        place(r, k);
-#pragma unroll
-        for (int c = 0; c < NC; ++c) {
-            const int64_t pr = row0 + r + prow(c);
-            const int64_t pkk = k0 + k + pk(c);
-            const bool inside = KC ? (pr < rows && pkk + V <= kdim) : (pkk < kdim && pr + V <= rows);
-            const bool outside = pr >= rows || pkk >= kdim;
-            if (inside) {
-                reg[c] = *reinterpret_cast<const mem_t*>(KC ? p + pr * ld + pkk : p + pkk * ld + pr);
-            } else if (outside) {
-#pragma unroll
-                for (int e = 0; e < V; ++e) reg[c][e] = T(0);
-            } else {
-#pragma unroll
-                for (int e = 0; e < V; ++e) {
-                    const int64_t gr = pr + (KC ? 0 : e);
-                    const int64_t gk = pkk + (KC ? e : 0);
-                    const bool ok = gr < rows && gk < kdim;
-                    const T x = *(ok ? (KC ? p + gr * ld + gk : p + gk * ld + gr) : p);
-                    reg[c][e] = ok ? x : T(0);
-                }
-            }
-        }
-    }
-
-    __device__ __forceinline__ void store(T* s) const {
-        int r, k;
-        place(r, k);
-        T* dst = KC ? (s + r * PITCH + k) : (s + k * PITCH + r);
-#pragma unroll
-        for (int c = 0; c < NC; ++c)
-            *reinterpret_cast<vec_t*>(KC ? dst + pk(c) : dst + pk(c) * PITCH + prow(c)) = reg[c];
-    }
-
-    // After a clamped load<false> of an RC operand: each piece that was
-    // started early is moved down by its overshoot.
-    __device__ __forceinline__ void align(int64_t row0, int64_t rows) {
-        if (KC) return;
-        int r, k;
-        place(r, k);
-#pragma unroll
-        for (int c = 0; c < NC; ++c) {
-            const int64_t over = row0 + r + prow(c) + V - rows;  // <= 0: not clamped; >= V: no row inside
-            const int s = over > 0 ? (int)over : 0;
-            vec_t x = reg[c];
-            if constexpr (V == 4) {
-                const vec_t y = (s & 2) ? vec_t{x[2], x[3], x[0], x[1]} : x;
-                reg[c] = (s & 1) ? vec_t{y[1], y[2], y[3], y[0]} : y;
-            } else {
-                reg[c] = (s & 1) ? vec_t{x[1], x[0]} : x;
-            }
-        }
-    }
-
-    // The four k values (MFMA steps 0..3 of 16-k pass kk) this lane feeds for
-    // the 16-row block at rb.
-    __device__ __forceinline__ static void frag(const T* s, int rb, int lane, int kk, T out[4]) {
-        const int r = rb + (lane & 15);
-        const int g = lane >> 4;
-        if (KC) {
-            typedef typename VecN<T, 4>::type v4_t;
-            const v4_t x = *reinterpret_cast<const v4_t*>(s + r * PITCH + 16 * kk + 4 * g);
-#pragma unroll
-            for (int st = 0; st < 4; ++st) out[st] = x[st];
-        } else {
-#pragma unroll
-            for (int st = 0; st < 4; ++st) out[st] = s[(16 * kk + 4 * g + st) * PITCH + r];
-        }
-    }
-};
 
 // FULL: M and N are multiples of the tile (no row or column clamping).
 template <typename T, int BM, int BN, int FM, int FN, bool TA, bool TB, bool FULL, bool DOT, int NBUF, int BK>
@@ -1213,31 +1045,30 @@ static int launch_tile(GemmArgs& g, bool ta, bool tb, hipStream_t st) {
     return check_launch("tt_gemm");
 }
 
-// Small problems: 32 x 32 tiles (four 16 x 16 wave tiles) and one stage that
-// holds all of K, so a launch makes one round trip to memory instead of one
-// per 16-deep stage. Both operands k-contiguous (A not transposed, B
-// transposed), the layouts whose 32-row stage the staging supports. The k
-// order per output is the other tiles' (16-deep passes in order).
-template <typename T, int BK>
-static int launch_small(GemmArgs& g, hipStream_t st) {
-    g.tiles_m = (g.M + 31) / 32;
-    g.tiles_n = (g.N + 31) / 32;
-    const int64_t total = g.tiles_m * g.tiles_n * g.batch;
-    if (total > 0x7fffffffLL) return set_error(TT_UNSUPPORTED, "tt_gemm: %lld tiles exceed one launch", (long long)total);
-    const dim3 grid((unsigned)total), block(kThreads);
-    hipLaunchKernelGGL((gemm_kernel<T, 32, 32, 1, 1, false, true, false, false, 1, BK>), grid, block, 0, st, g);
-    return check_launch("tt_gemm");
-}
-
 template <typename T, bool DOT>
 static int gemm_typed(GemmArgs& g, bool ta, bool tb, hipStream_t st) {
     constexpr int V = Vec16<T>::n;
-    // One 32 x 32 tile per batch entry and K within one deep stage (the
-    // DF-MP2 pair block 'ap,bp->ab' of config 1: 32 x 32 x 96).
-    constexpr int64_t KS = 512 / sizeof(T);  // 128 fp32, 64 fp64
-    if (!DOT && !ta && tb && g.M <= 32 && g.N <= 32 && g.K <= KS) {
-        if (g.K <= KS / 2) return launch_small<T, KS / 2>(g, st);
-        return launch_small<T, KS>(g, st);
+    // Grids too small for the wide tiles: 32 x 32 tiles (tt_gemm_small.hip).
+    // fp64: fewer than 192 tiles of 64 x 128 (three quarters of the CUs): at
+    // 180 tiles (1100 x 1200 x 500) 39.5 against 40.9 us on the direct-B kernel,
+    // at 160 34.1 against 39.9, at 209 (1200 x 1300 x 500) 44.7 against 41.3, at
+    // 242 (1400^2 x 700) 64 against 57. fp32: fewer than 384 tiles of 64 x 64
+    // (256 tiles, 1000^3: 31 against 54 us on the 64 x 128 tiles; 368, 1024 x
+    // 1455 x 315: 17 against 20; 512, 2000 x 1000 x 200: 17.3 against 15.3);
+    // where 32-wide tiles leave out an eighth of the 64-wide ones' padding, up
+    // to 1024 tiles of 64 x 64 (64 x 200 x 200 x 400: 33.5 against 38 us; past
+    // that the wide tiles' rate counts more: 80 x 200000 x 300 164 against 153
+    // us); and where they leave out a third of it (100000 x 16 x 300: 31
+    // against 58 us, 21 x 94905 x 171: 24 against 41 us).
+    if constexpr (!DOT) {
+        constexpr int64_t WN = sizeof(T) == 8 ? 128 : 64, FEW = sizeof(T) == 8 ? 192 : 384;
+        auto pad = [](int64_t n, int64_t t) { return (n + t - 1) / t * t; };
+        const int64_t wide = pad(g.M, 64) * pad(g.N, WN) * g.batch;
+        const int64_t narrow = pad(g.M, 32) * pad(g.N, 32) * g.batch;
+        bool small = wide < FEW * 64 * WN;
+        if constexpr (sizeof(T) == 4)
+            small = small || (wide <= (int64_t)1024 * 64 * 64 && 8 * wide > 9 * narrow) || 2 * wide >= 3 * narrow;
+        if (small) return gemm_small_launch(sizeof(T) == 8 ? TT_F64 : TT_F32, ta, tb, g, st);
     }
     // fp64: A through LDS, B straight into the MFMA registers
     // (gemm_directb_kernel above), non-temporal when B is read once (M <= 64
@@ -1256,13 +1087,15 @@ static int gemm_typed(GemmArgs& g, bool ta, bool tb, hipStream_t st) {
     // (160000 x 16384 x 800, B k-contiguous) 66.2-66.4 against 67.9-68.0 ms,
     // 16900 x 900 x 450 (both extents ragged) 0.31 against 0.35 ms, the sum
     // equal to 2e-15 (another order of the per-tile sums).
-    // What is left for fp64 (N = 1, or a transposed A of one row: no whole
-    // 16-byte piece along a row-contiguous operand) runs on the LDS tiles.
+    // What is left for fp64 (N = 1 or a transposed A of one row: no whole
+    // 16-byte piece along a row-contiguous operand) runs on the 32 x 32 tiles
+    // (100000 x 1 x 300 51 against 118 us on 256 x 64 LDS tiles), with the dot epilogue
+    // on the 64 x 128 LDS tiles.
     if constexpr (sizeof(T) == 8) {
         if (g.N >= V && (!ta || g.M >= V))
             return launch_directb<T, DOT>(g, ta, tb, g.M <= 64 && (g.batch == 1 || g.sB != 0), st);
-        if (g.M > 64) return launch_tile<T, 256, 64, 4, 4, DOT>(g, ta, tb, st);
-        return launch_tile<T, 64, 128, 2, 4, DOT>(g, ta, tb, st);
+        if constexpr (!DOT) return gemm_small_launch(TT_F64, ta, tb, g, st);
+        else return launch_tile<T, 64, 128, 2, 4, DOT>(g, ta, tb, st);
     } else {
         // fp32 direct-B on 64 x 256 tiles (four 16-column MFMA blocks per wave, so
         // a lane's B piece is still 16 bytes): within 1-2% of the LDS-staged
