@@ -86,3 +86,34 @@ def test_gemm_dot_unaligned_ragged(hip, dt, ta, tb, M, N, K):
     X = torch.bmm(A, B)
     scale = float((X.abs() * E.abs()).sum())
     assert abs(float(out) - float((X * E).sum())) <= TOL[dt] * scale
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("M,N,K", [(33, 47, 21), (500, 700, 37), (1030, 1025, 18), (2050, 2049, 17), (1, 1, 16), (17, 3, 100)])
+def test_gemm_dd_tiles(hip, ta, tb, M, N, K):
+    """The double-double GEMM's tiles (chosen by the grid they give): every
+    shape against float64, and bitwise against the same rows computed in
+    blocks of 40, whose grids take smaller tiles: the order of an output's
+    sums does not depend on the tile."""
+    from trntensor_amd.hip import engine
+
+    g = torch.Generator().manual_seed(M + N + K)
+    A = torch.randn(1, M, K, generator=g, dtype=torch.float64)
+    B = torch.randn(1, K, N, generator=g, dtype=torch.float64)
+    dt = torch.float64
+    sa, sb = A.transpose(1, 2) if ta else A, B.transpose(1, 2) if tb else B
+    lda, ldb = sa.shape[2] + 1, sb.shape[2] + 1
+    Ab, sA, _ = embed(sa, lda, 1, dt)
+    Bb, sB, _ = embed(sb, ldb, 1, dt)
+    with engine.accumulation("dd"):
+        Db, sD, D = embed(torch.full((1, M, N), float("nan")), N + 1, 1, dt)
+        engine.gemm(ta, tb, M, N, K, Ab, lda, sA, Bb, ldb, sB, Db, N + 1, sD, 1, 1.0, 0.0, None, 0, 0, a_off=1,
+                    b_off=1, d_off=1)
+        for m in range(0, min(M, 200), 40):
+            h = min(40, M - m)
+            P = torch.empty(h, N, dtype=dt, device="cuda")
+            engine.gemm(ta, tb, h, N, K, Ab, lda, sA, Bb, ldb, sB, P, N, 0, 1, 1.0, 0.0, None, 0, 0,
+                        a_off=1 + (m if ta else m * lda), b_off=1)
+            assert torch.equal(P, D[0, m : m + h])
+    assert normwise(D.cpu(), torch.bmm(A, B)) <= TOL[dt]
+    assert int(torch.isnan(Db).sum()) == Db.numel() - M * N

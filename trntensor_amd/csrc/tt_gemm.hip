@@ -957,8 +957,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_directb_stream_kernel(GemmAr
     }
 }
 
-// Compute units of the current device (cached per device).
-static int device_cus() {
+int device_cus() {
     static int cus[64];
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;

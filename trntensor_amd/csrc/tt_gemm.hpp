@@ -28,6 +28,8 @@ struct GemmArgs {
     double* partial;
 };
 
+// Compute units of the current device (cached per device).
+int device_cus();
 // tt_gemm after argument checks (store epilogue).
 int gemm_dispatch(int dtype, bool ta, bool tb, GemmArgs& g, hipStream_t st);
 // Double-double GEMM (dtype TT_F64_DD) on the vector ALUs; same arguments.
