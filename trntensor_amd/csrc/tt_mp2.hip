@@ -37,7 +37,20 @@ constexpr int kMp2Tile = 64;
 // 3.961 ms, naux 2400 fp64 15.33 against 15.42 ms, nocc 128 / nvir 640 /
 // naux 2400 243.0 against 243.2 ms (groups of 8: 7.401, 3.960, 15.26, 241.8;
 // of 64: 7.389, 3.902, 15.31, 243.4).
-constexpr int kMp2PairGroup = 16;
+constexpr int64_t kMp2PairGroup = 16;
+// Up to 1024 pairs one group is an XCD's share of the pairs: its short
+// diagonal units then end the launch instead of ending every group. Same box,
+// alternating, against groups of 16: nocc 21, nvir 150, naux 560 fp64 153
+// against 176 us, fp32 87 against 90; nocc 18, nvir 131 fp64 110 against 145;
+// nocc 30, nvir 200, naux 600 fp64 521 against 545, fp32 280 against 296; nocc
+// 40, nvir 257 fp64 714 against 729; with 2080 pairs and more equal to 1.5%
+// slower.
+static int mp2_pair_group(int64_t nocc) {
+    const int64_t npairs = nocc * (nocc + 1) / 2;
+    if (npairs > 1024) return (int)kMp2PairGroup;
+    const int64_t share = (npairs + kNumXcd - 1) / kNumXcd;
+    return (int)(share > 0 ? share : 1);
+}
 #ifndef TT_MP2_STAGE_K
 #define TT_MP2_STAGE_K 16
 #endif
@@ -50,21 +63,19 @@ constexpr int kMp2StageK = TT_MP2_STAGE_K;  // k per LDS stage
 // g = lane / 16 the k index E g + s, so a lane's E values per stage are
 // adjacent in LDS and one vector read feeds E MFMAs.
 //
-// AW is the global access width in elements: each thread's E values are
-// E / AW loads of AW consecutive elements. The launcher picks the widest AW
-// (16, 8 or 4 bytes) that every row start (a multiple of naux from B's base)
-// keeps naturally aligned, so rows of any naux take the branch-free
-// interior loop; only the access width narrows.
-template <typename T, int BK, int AW>
+// Global accesses are 16 bytes wide at the element's own alignment, so rows
+// of any naux from any base address take them.
+template <typename T, int BK>
 struct Panel {
     static constexpr int E = BK / 4;  // elements per thread, = MFMA steps per stage
+    static constexpr int AW = 16 / sizeof(T);  // elements per global access
     static constexpr int NP = E / AW;  // global loads per thread per stage
     static constexpr int PITCH = BK + 16 / sizeof(T);
     static constexpr int ELEMS = kMp2Tile * PITCH;
     static_assert(BK == 8 || BK == 16, "stage depth");
-    static_assert(AW >= 1 && E % AW == 0 && AW * sizeof(T) <= 16, "access width");
+    static_assert(E % AW == 0, "access width");
     typedef typename VecN<T, E>::type vec_t;
-    typedef typename VecN<T, AW>::type piece_t;
+    typedef T piece_t __attribute__((ext_vector_type(16 / sizeof(T)), aligned(sizeof(T))));
 
     vec_t reg;
 
@@ -130,6 +141,7 @@ struct Mp2Args {
     int64_t npq;     // nblk * (nblk + 1) / 2
     int64_t first;   // first work unit of this launch
     int64_t ntasks;  // work units in this launch (of npq * nocc * (nocc + 1) / 2)
+    int group;       // occupied pairs per group of the unit order
 };
 
 // Index of (x, y), x <= y < n, in row-major upper-triangle order -> (x, y).
@@ -143,21 +155,39 @@ __device__ __forceinline__ void tri_decode(int64_t idx, int n, int& x, int& y) {
     y = r + (int)idx;
 }
 
-// K loop of one work unit: X = P0 Q0^T and, if NEED_Y, Y = P2 Q3^T, BK k per
+// What a unit forms and how its four waves share it. A last block of at most
+// 32 rows takes the narrow forms: with the full ones half of the waves (three
+// of four for a diagonal block) would have no columns, and the unit would
+// hold its slot on the CU as long as a full one. us, with the idle waves only
+// skipping their MFMAs / with the narrow forms: nocc 21, nvir 150, naux 560
+// fp32 87 / 79, fp64 153 / 140; nocc 18, nvir 131 104 / 90 fp64; nocc 30, nvir
+// 200, naux 600 312 / 279 fp32; nocc 28, nvir 19, naux 748 27 / 21 fp32, 41 /
+// 32 fp64.
+enum Mp2Mode {
+    MP2_XY,         // X and Y: waves 0, 1 X, waves 2, 3 Y, 64 rows x 32 columns each
+    MP2_X,          // X only: 32 x 32 quadrants
+    MP2_XY_NARROW,  // X and Y, at most 32 columns: 32 rows x 32 columns each
+    MP2_X_NARROW,   // X only, at most 32 rows and columns: 16 x 16 quadrants
+};
+
+// K loop of one work unit: X = P0 Q0^T and, with Y, Y = P2 Q3^T, BK k per
 // stage. Stages whose successor is interior run in the first loop with
 // unconditional prefetch; the rest (edge rows, the K remainder, the last
 // stage) run in the second loop.
-template <typename T, int BK, int AW, bool NEED_Y>
-__device__ __forceinline__ void mp2_kloop(T* lds_base, const T* base0, const T* base1,
+template <typename T, int BK, Mp2Mode MODE, bool TAIL>
+__device__ __forceinline__ void mp2_kloop(int wave, T* lds_base, const T* base0, const T* base1,
                                           const T* base2, const T* base3, int rows_p, int rows_q, int64_t naux,
                                           typename Mfma<T>::acc_t (&X)[2][2], typename Mfma<T>::acc_t (&Y)[2][2]) {
     typedef Mfma<T> MF;
-    typedef Panel<T, BK, AW> PN;
+    typedef Panel<T, BK> PN;
     constexpr int KS = PN::E;
     const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const int wr = (wave >> 1) * 32;
-    const int wc = (wave & 1) * 32;
+    constexpr int AW = PN::AW;
+    constexpr bool NEED_Y = MODE == MP2_XY || MODE == MP2_XY_NARROW;
+    constexpr bool NARROW = MODE == MP2_XY_NARROW || MODE == MP2_X_NARROW;
+    constexpr int QS = NARROW ? 16 : 32;  // X only: rows and columns per wave
+    const int wr = (wave >> 1) * QS;
+    const int wc = (wave & 1) * QS;
     const int64_t nk = (naux + BK - 1) / BK;
     // Stages 0 .. nfull-1 are interior (all BK k in range). Ragged blocks (fewer than 64 rows) take this loop too, their missing
     // rows reading the block's last row: config 4's shape with nvir 300
@@ -184,7 +214,8 @@ __device__ __forceinline__ void mp2_kloop(T* lds_base, const T* base0, const T* 
     // panels 0 and 2 are staged, at lds_base + (2 b + k / 2) * ELEMS.
     auto lds = [&](int b, int k) -> T* { return lds_base + (DQ ? 2 * b + (k >> 1) : 4 * b + k) * PN::ELEMS; };
     const int qmat = wave >> 1;
-    const int qch = (wave & 1) * 32;
+    const int qch = NARROW ? 0 : (wave & 1) * 32;
+    const int prow = NARROW ? (wave & 1) * 32 : 0;  // first row of the wave's row blocks
     const T* qbase = qmat ? base3 : base1;
     typename PN::vec_t fq[2];
     auto qload = [&](int b, int64_t k0, auto fast) __attribute__((always_inline)) {
@@ -240,9 +271,10 @@ __device__ __forceinline__ void mp2_kloop(T* lds_base, const T* base0, const T* 
             // of both (fp64 166 -> 158 VGPRs; config 4 7.86-7.87 against 7.93
             // ms; fp32 measured the same at 104 VGPRs).
             const T* rp = lds(buf, qmat ? 2 : 0);
-            typename PN::vec_t fr[4];
+            constexpr int FR = NARROW ? 2 : 4;  // 16-row blocks per wave
+            typename PN::vec_t fr[FR];
 #pragma unroll
-            for (int a = 0; a < 4; ++a) fr[a] = PN::frag(rp, 16 * a, lane);
+            for (int a = 0; a < FR; ++a) fr[a] = PN::frag(rp, prow + 16 * a, lane);
 #pragma unroll
             for (int b = 0; b < 2; ++b) {
 #pragma unroll
@@ -250,7 +282,7 @@ __device__ __forceinline__ void mp2_kloop(T* lds_base, const T* base0, const T* 
 #pragma unroll
                     for (int a = 0; a < 2; ++a) {
                         X[a][b] = MF::mma(fr[a][st], fq[b][st], X[a][b]);
-                        Y[a][b] = MF::mma(fr[a + 2][st], fq[b][st], Y[a][b]);
+                        if constexpr (!NARROW) Y[a][b] = MF::mma(fr[a + 2][st], fq[b][st], Y[a][b]);
                     }
                 if (next == 1) qload(b, k0n, std::true_type{});
                 else if (next == 2) qload(b, k0n, std::false_type{});
@@ -258,17 +290,18 @@ __device__ __forceinline__ void mp2_kloop(T* lds_base, const T* base0, const T* 
             return;
         }
         // X only (i = j or p = q): quadrants, both panels through LDS.
-        typename PN::vec_t f0[2], f1[2];
+        constexpr int NQ = NARROW ? 1 : 2;  // 16-row and 16-column blocks per wave
+        typename PN::vec_t f0[NQ], f1[NQ];
 #pragma unroll
-        for (int a = 0; a < 2; ++a) f0[a] = PN::frag(lds(buf, 0), wr + 16 * a, lane);
+        for (int a = 0; a < NQ; ++a) f0[a] = PN::frag(lds(buf, 0), wr + 16 * a, lane);
 #pragma unroll
-        for (int b = 0; b < 2; ++b) f1[b] = PN::frag(lds(buf, 1), wc + 16 * b, lane);
+        for (int b = 0; b < NQ; ++b) f1[b] = PN::frag(lds(buf, 1), wc + 16 * b, lane);
 #pragma unroll
         for (int st = 0; st < KS; ++st)
 #pragma unroll
-            for (int a = 0; a < 2; ++a)
+            for (int a = 0; a < NQ; ++a)
 #pragma unroll
-                for (int b = 0; b < 2; ++b) X[a][b] = MF::mma(f0[a][st], f1[b][st], X[a][b]);
+                for (int b = 0; b < NQ; ++b) X[a][b] = MF::mma(f0[a][st], f1[b][st], X[a][b]);
     };
 
     // One LDS stage buffer and one register prefetch set: while stage k is
@@ -282,6 +315,21 @@ __device__ __forceinline__ void mp2_kloop(T* lds_base, const T* base0, const T* 
     // 0.7% (config 4, same box, alternating: 7.65 against 7.70 ms; fp32 4.10
     // against 4.00 ms), so neither dtype raises it.
     if (nk == 0) return;
+    // X only: a wave whose columns or rows all lie past the block's end
+    // only helps stage: the same loads, stores and barriers, no fragments and
+    // no MFMAs, so its SIMD's MFMA pipe serves the other workgroups. Its
+    // accumulators stay zero and the energy loop skips them.
+    if (TAIL && MODE == MP2_X && (wc >= rows_q || wr >= rows_p)) {
+        for (int64_t k = 0; k < nk; ++k) {
+            if (k < nfull) load(k * BK, std::true_type{});
+            else load(k * BK, std::false_type{});
+            if (k > 0) __syncthreads();
+            store(0);
+            __syncthreads();
+        }
+        __syncthreads();  // the live waves' barrier after their last stage
+        return;
+    }
     if (nfull > 0) {
         load(0, std::true_type{});
         if (DQ) qload(0, 0, std::true_type{}), qload(1, 0, std::true_type{});
@@ -304,7 +352,7 @@ __device__ __forceinline__ void mp2_kloop(T* lds_base, const T* base0, const T* 
             // after the 4th and 8th MFMA instead: 4.11-4.13 ms; the same
             // spacing in fp64 (eight loads): -0.6% at naux 1200, +0.7% at 2400.
             constexpr int NL = 4 * PN::NP;  // loads per thread per stage
-            constexpr int NM = 8 * KS;      // MFMAs per wave per stage
+            constexpr int NM = (NARROW ? 4 : 8) * KS;  // MFMAs per wave per stage
 #pragma unroll
             for (int l = 0; l < NL; ++l) {
                 __builtin_amdgcn_sched_group_barrier(0x008, NM / NL, 0);
@@ -322,23 +370,28 @@ __device__ __forceinline__ void mp2_kloop(T* lds_base, const T* base0, const T* 
         compute(0, (kt + 1) * BK, more ? 2 : 0);
         __builtin_amdgcn_sched_barrier(0);
         __syncthreads();
-        if (more) store(0);
-        __syncthreads();
+        if (more) {
+            store(0);
+            __syncthreads();
+        }
     }
 }
 
-template <typename T, int BK, int AW>
+// TAIL: the last virtual block has at most 32 rows (the narrow forms exist; the
+// kernel without them keeps the registers and schedule of the full forms:
+// nocc 64, nvir 320, naux 1200 fp64 0.6% faster).
+template <typename T, int BK, bool TAIL>
 __global__ __launch_bounds__(kMp2Threads) void mp2_energy_kernel(Mp2Args g) {
     typedef Mfma<T> MF;
     typedef typename MF::acc_t acc_t;
-    typedef Panel<T, BK, AW> PN;
+    typedef Panel<T, BK> PN;
 
     __shared__ __attribute__((aligned(16))) T lds[1][4][PN::ELEMS];
     __shared__ double red[4];
 
     const int64_t local = xcd_remap(blockIdx.x, g.ntasks);
     const int64_t task = g.first + local;
-    // Unit order: groups of kMp2PairGroup occupied pairs; within a group, the
+    // Unit order: groups of g.group occupied pairs; within a group, the
     // off-diagonal units (p < q) of all its pairs first, pair-major and
     // row-major over p < q, then its diagonal units (p = q). A diagonal unit
     // issues half the MFMAs per stage and runs ahead of the off-diagonal
@@ -348,15 +401,15 @@ __global__ __launch_bounds__(kMp2Threads) void mp2_energy_kernel(Mp2Args g) {
     int64_t pair, u;
     {
         const int64_t npairs = (int64_t)g.nocc * (g.nocc + 1) / 2;
-        const int64_t grp = task / (kMp2PairGroup * g.npq);
-        const int64_t gp = min((int64_t)kMp2PairGroup, npairs - grp * kMp2PairGroup);  // pairs in this group
-        const int64_t r = task - grp * kMp2PairGroup * g.npq;
+        const int64_t grp = task / ((int64_t)g.group * g.npq);
+        const int64_t gp = min((int64_t)g.group, npairs - grp * g.group);  // pairs in this group
+        const int64_t r = task - grp * (int64_t)g.group * g.npq;
         if (r < gp * noff) {
-            pair = grp * kMp2PairGroup + r / noff;
+            pair = grp * g.group + r / noff;
             u = r % noff;
         } else {
             const int64_t r2 = r - gp * noff;
-            pair = grp * kMp2PairGroup + r2 / g.nblk;
+            pair = grp * g.group + r2 / g.nblk;
             u = noff + r2 % g.nblk;
         }
     }
@@ -384,7 +437,10 @@ __global__ __launch_bounds__(kMp2Threads) void mp2_energy_kernel(Mp2Args g) {
     const T* base3 = B + ((int64_t)i * nvir + (int64_t)q * kMp2Tile) * g.naux;
 
     const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
+    // As a scalar, the wave index frees the fp32 TAIL kernel the registers of a
+    // fifth workgroup per CU (nocc 21, nvir 150, naux 555: 81 against 87 us);
+    // the other kernel is 1.5% slower that way (config 4 fp32).
+    const int wave = TAIL ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : (int)(threadIdx.x >> 6);
     const int wr = (wave >> 1) * 32;  // quadrant row offset (a within p)
     const int wc = (wave & 1) * 32;   // quadrant col offset (b within q)
 
@@ -397,15 +453,54 @@ __global__ __launch_bounds__(kMp2Threads) void mp2_energy_kernel(Mp2Args g) {
             Y[a][b] = acc_t{0, 0, 0, 0};
         }
 
-    if (ymode == 0)
-        mp2_kloop<T, BK, AW, true>(&lds[0][0][0], base0, base1, base2, base3, rows_p, rows_q, g.naux, X, Y);
-    else
-        mp2_kloop<T, BK, AW, false>(&lds[0][0][0], base0, base1, base2, base3, rows_p, rows_q, g.naux, X, Y);
+    const bool narrow = TAIL && rows_q <= 32 && ymode != 1;
+    if (ymode == 0 && !narrow)
+        mp2_kloop<T, BK, MP2_XY, TAIL>(wave, &lds[0][0][0], base0, base1, base2, base3, rows_p, rows_q, g.naux, X, Y);
+    else if (TAIL && ymode == 0)
+        mp2_kloop<T, BK, MP2_XY_NARROW, TAIL>(wave, &lds[0][0][0], base0, base1, base2, base3, rows_p, rows_q, g.naux, X, Y);
+    else if (!narrow)
+        mp2_kloop<T, BK, MP2_X, TAIL>(wave, &lds[0][0][0], base0, base1, base2, base3, rows_p, rows_q, g.naux, X, Y);
+    else if (TAIL)
+        mp2_kloop<T, BK, MP2_X_NARROW, TAIL>(wave, &lds[0][0][0], base0, base1, base2, base3, rows_p, rows_q, g.naux, X, Y);
 
     const int lg = lane >> 4;
-    // Rows and columns of the quadrant the energy loop below reads from X and Y.
-    int rb = wr, cb0 = wc;
-    if (ymode == 0) {
+    // Rows and columns the energy loop below reads from X and Y, and how many
+    // 16-row and 16-column blocks of them.
+    int rb = wr, cb0 = wc, na = 2, nb = 2;
+    if (ymode == 0 && narrow) {
+        // Each X wave holds 32 rows of X (in X), the Y wave of the same rows
+        // those of Y (in X too): the X wave keeps its first 16 rows, the Y wave
+        // its last 16, and each hands the other half over.
+        const int mat = wave >> 1;
+        constexpr int TP = 33;
+        T* xs = &lds[0][0][0] + (wave & 1) * 16 * TP;  // X, last 16 of the 32 rows
+        T* ys = xs + 32 * TP;                          // Y, first 16
+        static_assert(64 * TP <= 4 * PN::ELEMS, "exchange fits in the staging buffers");
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int o = MF::row(lg, r) * TP + 16 * b + (lane & 15);
+                if (mat == 0) xs[o] = X[1][b][r];
+                else ys[o] = X[0][b][r];
+            }
+        __syncthreads();
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int o = MF::row(lg, r) * TP + 16 * b + (lane & 15);
+                if (mat == 0) {
+                    Y[0][b][r] = ys[o];
+                } else {
+                    Y[0][b][r] = X[1][b][r];
+                    X[0][b][r] = xs[o];
+                }
+            }
+        rb = (wave & 1) * 32 + mat * 16;
+        cb0 = 0;
+        na = 1;
+    } else if (ymode == 0) {
         // The K loop left each X wave with X rows 0-63 of its columns
         // and each Y wave with Y rows 0-63 of the same columns. The X wave
         // keeps rows 0-31 and hands rows 32-63 to the Y wave, which keeps its
@@ -441,7 +536,19 @@ __global__ __launch_bounds__(kMp2Threads) void mp2_energy_kernel(Mp2Args g) {
         rb = mat ? 32 : 0;
         cb0 = ch;
     }
-    if (ymode == 2) {
+    if (ymode == 2 && narrow) {
+        // Y = X^T through LDS, 16 x 16 quadrants.
+        constexpr int TP = 33;
+        T* tr = &lds[0][0][0];
+        rb = (wave >> 1) * 16;
+        cb0 = (wave & 1) * 16;
+        na = nb = 1;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) tr[(rb + MF::row(lg, r)) * TP + cb0 + (lane & 15)] = X[0][0][r];
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 4; ++r) Y[0][0][r] = tr[(cb0 + (lane & 15)) * TP + rb + MF::row(lg, r)];
+    } else if (ymode == 2) {
         // Y = X^T through LDS (the staging buffers are free after the last barrier).
         constexpr int TP = kMp2Tile + 1;
         T* tr = &lds[0][0][0];
@@ -488,14 +595,14 @@ __global__ __launch_bounds__(kMp2Threads) void mp2_energy_kernel(Mp2Args g) {
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
         const int cb = cb0 + 16 * b + (lane & 15);
-        const bool okb = cb < rows_q;
+        const bool okb = cb < rows_q && b < nb;
         const T e_b = e_bv[b];
 #pragma unroll
         for (int a = 0; a < 2; ++a) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int ra = rb + 16 * a + MF::row(lg, r);
-                if (okb && ra < rows_p) {
+                if (okb && ra < rows_p && a < na) {
                     const T e_a = e_av[a][r];
                     const T x = X[a][b][r];
                     const T y = ymode == 1 ? x : Y[a][b][r];
@@ -533,30 +640,22 @@ __global__ void zero_double_kernel(double* p) {
     if (threadIdx.x == 0) p[0] = 0.0;
 }
 
-// Largest of 16 / sizeof(T), ..., 2, 1 elements such that B's base and every
-// row start (multiples of naux elements from it) are aligned to that many
-// elements' bytes.
-static int mp2_access_width(size_t elem, int64_t naux, const void* B) {
-    int aw = (int)(16 / elem);
-    while (aw > 1 && ((naux % aw) != 0 || (reinterpret_cast<uintptr_t>(B) % (aw * elem)) != 0)) aw >>= 1;
-    return aw;
-}
-
 static int64_t mp2_ntasks(int64_t nocc, int64_t nvir) {
     const int64_t nblk = (nvir + kMp2Tile - 1) / kMp2Tile;
     return (nblk * (nblk + 1) / 2) * (nocc * (nocc + 1) / 2);
 }
 
 // Workspace layout: the per-unit partials (plus one double), then, when naux
-// is not a multiple of the stage depth, a copy of B whose rows are padded
-// with zeros to mp2_pitch(naux) elements.
+// is not a multiple of the stage depth, room for a copy of B whose rows are
+// padded with zeros to mp2_pitch(naux) elements. The copy is made where each
+// row is read often enough (mp2_copy_pays).
 //
 // The stages of a row start at multiples of 16 elements from the row start.
 // With naux a multiple of 16 (and B's base so aligned) every stage is a whole
 // 128-byte (fp64) or 64-byte (fp32) aligned chunk; otherwise each straddles
-// cache lines and the kernel runs 5-7% slower (nocc 64, nvir 320: naux 1199
-// fp64 8.58 ms against 8.06 ms on the padded copy, which itself takes
-// 0.07 ms; fp32 4.38 against 4.13 + 0.03 ms). The zero columns add nothing
+// cache lines (16-byte accesses at the element's alignment): nocc 64, nvir 320,
+// naux 1199 fp64 7.70 against 7.55 ms on the padded copy, which itself takes
+// 0.07 ms; fp32 4.07 against 3.93 ms. The zero columns add nothing
 // to any product, and the unpadded kernel masks the same columns to zero in
 // its last stage, so both give the same energy, bitwise.
 static size_t mp2_partials_bytes(int64_t nocc, int64_t nvir) {
@@ -573,6 +672,13 @@ static size_t mp2_pad_bytes(int dtype, int64_t nocc, int64_t nvir, int64_t naux)
     if (b > (unsigned __int128)(SIZE_MAX / 4)) return SIZE_MAX / 4;
     return (((size_t)b + 255) / 256) * 256;
 }
+
+// Whether the padded copy pays: a row of B is read about nocc * nvir / 64
+// times, the copy costs one pass over B. us on B as given / with the copy,
+// fp32, fp64: nocc 21, nvir 150, naux 555 (nocc * nvir 3150) 85 / 93, 145 /
+// 155; 30, 200, 600 padded to 608 (6000) 280 / 281, 516 / 521; 44, 175, 653
+// (7700) 417 / 409, 770 / 770; 48, 295, 269 (14160) 606 / 588, 1134 / 1104.
+static bool mp2_copy_pays(int64_t nocc, int64_t nvir) { return nocc * nvir >= 7000; }
 
 // src (rows x naux, contiguous) -> dst (rows x pitch), zero in columns naux
 // and beyond. One workgroup per row (grid-stride); each thread forms V
@@ -607,7 +713,7 @@ static int mp2_typed(int64_t nocc, int64_t nvir, int64_t naux, const void* B, co
     // aligned, which the copy's 16-byte stores and the stage alignment need).
     const size_t part = mp2_partials_bytes(nocc, nvir);
     const size_t pad = mp2_pad_bytes(sizeof(T) == 4 ? TT_F32 : TT_F64, nocc, nvir, naux);
-    if (pad > 0 && ws_bytes >= part && ws_bytes - part >= pad && (reinterpret_cast<uintptr_t>(ws) & 255) == 0) {
+    if (pad > 0 && mp2_copy_pays(nocc, nvir) && ws_bytes >= part && ws_bytes - part >= pad && (reinterpret_cast<uintptr_t>(ws) & 255) == 0) {
         T* Bp = reinterpret_cast<T*>(static_cast<char*>(ws) + part);
         const int64_t rows = nocc * nvir, pitch = mp2_pitch(naux);
         hipLaunchKernelGGL(mp2_pad_rows_kernel<T>, dim3((unsigned)(rows < 65536 ? rows : 65536)), dim3(256), 0, st,
@@ -624,6 +730,7 @@ static int mp2_typed(int64_t nocc, int64_t nvir, int64_t naux, const void* B, co
     g.nvir = (int)nvir;
     g.nblk = (int)((nvir + kMp2Tile - 1) / kMp2Tile);
     g.npq = (int64_t)g.nblk * (g.nblk + 1) / 2;
+    g.group = mp2_pair_group(nocc);
     g.first = first;
     g.ntasks = count;
     double* w = static_cast<double*>(ws);
@@ -636,17 +743,11 @@ static int mp2_typed(int64_t nocc, int64_t nvir, int64_t naux, const void* B, co
         hipLaunchKernelGGL(zero_double_kernel, dim3(1), dim3(64), 0, st, w);
     }
     constexpr int BK = kMp2StageK;
-    // Widest access (elements) that keeps every row start naturally aligned.
-    const int aw = mp2_access_width(sizeof(T), naux, B);
     if (g.ntasks > 0) {
-        const dim3 grid((unsigned)g.ntasks), block(kMp2Threads);
-        constexpr int V = 16 / sizeof(T);
-        if (aw == V)
-            hipLaunchKernelGGL((mp2_energy_kernel<T, BK, V>), grid, block, 0, st, g);
-        else if (aw == 2)
-            hipLaunchKernelGGL((mp2_energy_kernel<T, BK, 2>), grid, block, 0, st, g);
+        if (nvir % kMp2Tile >= 1 && nvir % kMp2Tile <= 32)
+            hipLaunchKernelGGL((mp2_energy_kernel<T, BK, true>), dim3((unsigned)g.ntasks), dim3(kMp2Threads), 0, st, g);
         else
-            hipLaunchKernelGGL((mp2_energy_kernel<T, BK, 1>), grid, block, 0, st, g);
+            hipLaunchKernelGGL((mp2_energy_kernel<T, BK, false>), dim3((unsigned)g.ntasks), dim3(kMp2Threads), 0, st, g);
     }
     hipLaunchKernelGGL(mp2_finalize_kernel<T>, dim3(1), dim3(256), 0, st, (const double*)w,
                        det ? g.ntasks : (int64_t)1, static_cast<T*>(out));
