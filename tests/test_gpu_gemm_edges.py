@@ -117,3 +117,39 @@ def test_gemm_dd_tiles(hip, ta, tb, M, N, K):
             assert torch.equal(P, D[0, m : m + h])
     assert normwise(D.cpu(), torch.bmm(A, B)) <= TOL[dt]
     assert int(torch.isnan(Db).sum()) == Db.numel() - M * N
+
+
+# fp32 sizes whose grids take the 64 x 64, the pipelined 64 x 128 and the
+# pipelined 128 x 128 tile, ragged in both extents and in K (also K below one
+# stage, whole stages, and one element over).
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("M,N", [(2061, 2051), (1999, 3001), (4001, 4003), (2048, 3072), (4096, 3968)])
+@pytest.mark.parametrize("K", [31, 64, 65])
+def test_gemm_f32_wide_tiles(hip, ta, tb, M, N, K):
+    """Against float64 torch on the device, with C and alpha/beta, operands
+    and D in NaN buffers; and bitwise against the last rows computed in a
+    product of 40 rows (the 32 x 32 tiles)."""
+    from trntensor_amd.hip import engine
+
+    dt = torch.float32
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    A = torch.randn(1, M, K, generator=g, dtype=torch.float64, device="cuda").to(dt)
+    B = torch.randn(1, K, N, generator=g, dtype=torch.float64, device="cuda").to(dt)
+    C = torch.randn(1, M, N, generator=g, dtype=torch.float64, device="cuda").to(dt)
+    sa, sb = A.transpose(1, 2) if ta else A, B.transpose(1, 2) if tb else B
+    pad = M % 2  # aligned for the whole-tile shapes
+    lda, ldb = sa.shape[2] + pad, sb.shape[2] + pad
+    Ab, sA, _ = embed(sa, lda, pad, dt)
+    Bb, sB, _ = embed(sb, ldb, pad, dt)
+    Cb, sC, _ = embed(C, N + pad, pad, dt)
+    Db, sD, D = embed(torch.full((1, M, N), float("nan")), N + pad, pad, dt)
+    engine.gemm(ta, tb, M, N, K, Ab, lda, sA, Bb, ldb, sB, Db, N + pad, sD, 1, 1.5, 0.5, Cb[pad:], N + pad, sC,
+                a_off=pad, b_off=pad, d_off=pad)
+    ref = 1.5 * torch.matmul(A[0].double(), B[0].double()) + 0.5 * C[0].double()
+    assert float((D[0].double() - ref).abs().max() / ref.abs().max()) <= TOL[dt]
+    assert int(torch.isnan(Db).sum()) == Db.numel() - M * N
+    m = M - 40
+    P = torch.empty(40, N, dtype=dt, device="cuda")
+    engine.gemm(ta, tb, 40, N, K, Ab, lda, sA, Bb, ldb, sB, P, N, 0, 1, 1.5, 0.5, C[0, m:], N, 0,
+                a_off=pad + (m if ta else m * lda), b_off=pad)
+    assert torch.equal(P, D[0, m:])

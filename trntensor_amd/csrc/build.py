@@ -29,6 +29,7 @@ SOURCES = [
     "tt_gemm16.hip",
     "tt_gemm16_dma.hip",
     "tt_gemm_big.hip",
+    "tt_gemm_mid.hip",
     "tt_gemm_small.hip",
     "tt_mp2.hip",
     "tt_probe.hip",

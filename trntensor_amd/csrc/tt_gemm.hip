@@ -16,6 +16,8 @@
 // the k index 4 g + s for both operands, so a lane's four k values are
 // adjacent in the [row][k] layout and one 32-byte read feeds four MFMAs.
 #include <string.h>
+
+#include <algorithm>
 #include <type_traits>
 
 #include "tt_gemm.hpp"
@@ -1044,31 +1046,58 @@ static int launch_tile(GemmArgs& g, bool ta, bool tb, hipStream_t st) {
     return check_launch("tt_gemm");
 }
 
+// fp32 products (all kernels bitwise equal).
+static int gemm_f32(GemmArgs& g, bool ta, bool tb, hipStream_t st) {
+    const int64_t cus = device_cus();
+    // Both operands not transposed, whole 256 x 256 tiles in whole rounds of
+    // one tile per CU (at least 95% of the last round busy), without C or with
+    // K >= 1024: the 256 x 256 LDS tile (tt_gemm_big.hip). Same box,
+    // alternating, fraction of the fp32 peak against the 64 x 256 direct-B tile:
+    // 4096^3 with alpha/beta and C 0.93 against 0.88; 64 x 512^3 without C
+    // 0.834 against 0.806, 16 x 1024^3 with C 0.866 against 0.845. A partial
+    // last round loses (6144^2 x 2048, 2.25 rounds: 1.444 against 1.118 ms),
+    // and so does a short K with C, whose epilogue one wave per SIMD cannot
+    // hide (64 x 512^3 with C 0.785 against 0.801, 128 x 512^3 with C 0.760
+    // against 0.799).
+    if (gemm_big_f32_fits(ta, tb, g) && (!g.C || g.K >= 1024)) {
+        const int64_t tiles = (g.M / 256) * (g.N / 256) * g.batch;
+        const int64_t rounds = (tiles + cus - 1) / cus;
+        if (tiles >= cus && 100 * tiles >= 95 * rounds * cus) return gemm_big_f32_launch(g, st);
+    }
+    // Otherwise the tile with the least estimated time of the busiest CU: its
+    // tiles times their area, times the kernel's cost per output where every CU
+    // has many tiles (from 4096^3, 6144^2 x 2048, 1999 x 3001 x 1201 in the
+    // four layouts), times what one or two tiles on a CU lose because nothing
+    // covers their latencies (least on the pipelined tiles). us measured on
+    // direct-B 64 x 256 / 128 x 128 / 64 x 128 / 64 x 64 / 32 x 32: 2048 x 3072
+    // x 1216 161/158/136/144/163; 3001^2 x 1201 -/230/206/204/250; 1999 x 1501
+    // x 1201 NT -/81/84/72/81; 1400^2 x 3000 -/188/111/131/135; 30 x 300^2 x
+    // 1000 -/135/76/68/73; 1500^2 x 300 -/28/27/24/23; 1000^3 -/68/39/32/29;
+    // 150 x 2000 x 3000 -/186/105/86/52; 4000^2 x 1000 -/260/268/285/311; 64 x
+    // 786432 x 512 TN 452/787/470/535/623; 80 x 200000 x 300 TN
+    // -/156/150/170/160.
+    auto cost = [&](int64_t bm, int64_t bn, double per_output, double one, double two) {
+        const int64_t n = ((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn) * g.batch;
+        const int64_t rounds = (n + cus - 1) / cus;
+        return (double)(rounds * bm * bn) * per_output * (rounds == 1 ? one : rounds == 2 ? two : 1.0);
+    };
+    const bool rows_ok = !ta || g.M >= 4, cols_ok = tb || g.N >= 4;  // a 16-byte piece along a row-contiguous operand
+    const double never = 1e300;
+    const double direct = rows_ok && !tb && g.N % 256 == 0 ? cost(64, 256, 0.97, 1.1, 1.0) : never;
+    const double tall = rows_ok && cols_ok && g.K > 0 ? cost(128, 128, 1.0, 1.05, 1.0) : never;
+    const double mid = rows_ok && cols_ok && g.K > 0 ? cost(64, 128, 1.04, 1.05, 1.0) : never;
+    const double square = cost(64, 64, 1.1, 1.25, 1.1);
+    const double small = cost(32, 32, ta && !tb ? 1.5 : tb && !ta ? 1.25 : 1.35, 1.1, 1.1);
+    const double best = std::min({direct, tall, mid, square, small});
+    if (best == small) return gemm_small_launch(TT_F32, ta, tb, g, st);
+    if (best == square) return launch_tile<float, 64, 64, 2, 2, false, 1, 64>(g, ta, tb, st);
+    if (best == direct) return launch_directb<float, false>(g, ta, false, g.M <= 64 && (g.batch == 1 || g.sB != 0), st);
+    return gemm_mid_f32_launch(ta, tb, best == tall, g, st);
+}
+
 template <typename T, bool DOT>
 static int gemm_typed(GemmArgs& g, bool ta, bool tb, hipStream_t st) {
     constexpr int V = Vec16<T>::n;
-    // Grids too small for the wide tiles: 32 x 32 tiles (tt_gemm_small.hip).
-    // fp64: fewer than 192 tiles of 64 x 128 (three quarters of the CUs): at
-    // 180 tiles (1100 x 1200 x 500) 39.5 against 40.9 us on the direct-B kernel,
-    // at 160 34.1 against 39.9, at 209 (1200 x 1300 x 500) 44.7 against 41.3, at
-    // 242 (1400^2 x 700) 64 against 57. fp32: fewer than 384 tiles of 64 x 64
-    // (256 tiles, 1000^3: 31 against 54 us on the 64 x 128 tiles; 368, 1024 x
-    // 1455 x 315: 17 against 20; 512, 2000 x 1000 x 200: 17.3 against 15.3);
-    // where 32-wide tiles leave out an eighth of the 64-wide ones' padding, up
-    // to 1024 tiles of 64 x 64 (64 x 200 x 200 x 400: 33.5 against 38 us; past
-    // that the wide tiles' rate counts more: 80 x 200000 x 300 164 against 153
-    // us); and where they leave out a third of it (100000 x 16 x 300: 31
-    // against 58 us, 21 x 94905 x 171: 24 against 41 us).
-    if constexpr (!DOT) {
-        constexpr int64_t WN = sizeof(T) == 8 ? 128 : 64, FEW = sizeof(T) == 8 ? 192 : 384;
-        auto pad = [](int64_t n, int64_t t) { return (n + t - 1) / t * t; };
-        const int64_t wide = pad(g.M, 64) * pad(g.N, WN) * g.batch;
-        const int64_t narrow = pad(g.M, 32) * pad(g.N, 32) * g.batch;
-        bool small = wide < FEW * 64 * WN;
-        if constexpr (sizeof(T) == 4)
-            small = small || (wide <= (int64_t)1024 * 64 * 64 && 8 * wide > 9 * narrow) || 2 * wide >= 3 * narrow;
-        if (small) return gemm_small_launch(sizeof(T) == 8 ? TT_F64 : TT_F32, ta, tb, g, st);
-    }
     // fp64: A through LDS, B straight into the MFMA registers
     // (gemm_directb_kernel above), non-temporal when B is read once (M <= 64
     // and B not broadcast over the batch). Same box, alternating, bitwise
@@ -1090,47 +1119,28 @@ static int gemm_typed(GemmArgs& g, bool ta, bool tb, hipStream_t st) {
     // 16-byte piece along a row-contiguous operand) runs on the 32 x 32 tiles
     // (100000 x 1 x 300 51 against 118 us on 256 x 64 LDS tiles), with the dot epilogue
     // on the 64 x 128 LDS tiles.
+    // Grids too small for it take the 32 x 32 tiles (tt_gemm_small.hip): fewer
+    // than 192 tiles of 64 x 128 (three quarters of the CUs). At 180 tiles
+    // (1100 x 1200 x 500) 39.5 against 40.9 us on the direct-B kernel, at 160
+    // 34.1 against 39.9, at 209 (1200 x 1300 x 500) 44.7 against 41.3, at 242
+    // (1400^2 x 700) 64 against 57.
     if constexpr (sizeof(T) == 8) {
+        if (!DOT && ((g.M + 63) / 64) * ((g.N + 127) / 128) * g.batch < 192)
+            return gemm_small_launch(TT_F64, ta, tb, g, st);
         if (g.N >= V && (!ta || g.M >= V))
             return launch_directb<T, DOT>(g, ta, tb, g.M <= 64 && (g.batch == 1 || g.sB != 0), st);
         if constexpr (!DOT) return gemm_small_launch(TT_F64, ta, tb, g, st);
         else return launch_tile<T, 64, 128, 2, 4, DOT>(g, ta, tb, st);
-    } else {
-        // fp32 direct-B on 64 x 256 tiles (four 16-column MFMA blocks per wave, so
-        // a lane's B piece is still 16 bytes): within 1-2% of the LDS-staged
-        // tiles, ahead on short K (same box, alternating, bitwise equal: 4096^2 x
-        // 512 0.1345 against 0.1364 ms, 64 x 512^3 with alpha/beta and C 0.1397
-        // against 0.1414 ms, 4096^3 0.988 against 0.990 ms). Whole column tiles
-        // only: 3000 x 3000 x 1000 0.221 against 0.212 ms.
-        // fp32, both operands not transposed, whole 256 x 256 tiles in whole
-        // rounds of one tile per CU (at least 95% of the last round busy), without
-        // C or with K >= 1024: the 256 x 256 LDS tile (tt_gemm_big.hip), bitwise
-        // equal to the tiles below. Same box, alternating, fraction of the fp32
-        // peak against the 64 x 256 direct-B tile: 4096^3 with alpha/beta and C
-        // 0.93 against 0.88; 64 x 512^3 without C 0.834 against 0.806, 16 x
-        // 1024^3 with C 0.866 against 0.845. A partial last round loses (6144^2 x
-        // 2048, 2.25 rounds: 1.444 against 1.118 ms), and so does a short K with
-        // C, whose epilogue one wave per SIMD cannot hide (64 x 512^3 with C
-        // 0.785 against 0.801, 128 x 512^3 with C 0.760 against 0.799).
-        if constexpr (!DOT) {
-            if (gemm_big_f32_fits(ta, tb, g) && (!g.C || g.K >= 1024)) {
-                const int64_t tiles = (g.M / 256) * (g.N / 256) * g.batch, cus = device_cus();
-                const int64_t rounds = (tiles + cus - 1) / cus;
-                if (tiles >= cus && 100 * tiles >= 95 * rounds * cus) return gemm_big_f32_launch(g, st);
-            }
-            if (!tb && g.N % 256 == 0 && (!ta || g.M >= V))
-                return launch_directb<T, DOT>(g, ta, false, g.M <= 64 && (g.batch == 1 || g.sB != 0), st);
-        }
+    } else if constexpr (DOT) {
         if (g.M <= 64) return launch_tile<T, 64, 128, 2, 4, DOT>(g, ta, tb, st);
         if (g.N <= 64) return launch_tile<T, 256, 64, 4, 4, DOT>(g, ta, tb, st);
-        // Small grids: fewer than 448 128 x 128 tiles leave CUs idle; 64 x 128
-        // tiles double the grid (TFLOP/s against 128 x 128: 1024^3 41.9 against
-        // 21.9; 2000 x 3000 x 2000 77.2 against 59.5; 2048^3 112.4 against
-        // 90.8; at 484 tiles, 2816^3, 120.4 against 131.3). Results are
-        // identical (the k order per output does not depend on the tile).
+        // Fewer than 448 128 x 128 tiles leave CUs idle; 64 x 128 tiles double
+        // the grid.
         if (((g.M + 127) / 128) * ((g.N + 127) / 128) * g.batch < 448)
             return launch_tile<T, 64, 128, 2, 4, DOT>(g, ta, tb, st);
         return launch_tile<T, 128, 128, 4, 4, DOT>(g, ta, tb, st);
+    } else {
+        return gemm_f32(g, ta, tb, st);
     }
 }
 

@@ -45,6 +45,9 @@ int gemm16_dma_rows(bool ta, bool tb, int64_t K);
 void gemm16_dma_tile(bool ta, bool tb, int64_t M, int64_t N, int64_t K, int64_t batch, int& bm, int& bn);
 // fp32/fp64 on 32 x 32 tiles (tt_gemm_small.hip): any problem.
 int gemm_small_launch(int dtype, bool ta, bool tb, GemmArgs& g, hipStream_t st);
+// fp32 on pipelined 128 x 128 (tall) or 64 x 128 tiles (tt_gemm_mid.hip): K >= 1,
+// and M >= 4 with A transposed, N >= 4 with B not transposed.
+int gemm_mid_f32_launch(bool ta, bool tb, bool tall, GemmArgs& g, hipStream_t st);
 // fp32 on 256 x 256 tiles (tt_gemm_big.hip): whether it takes the problem,
 // and its launch.
 bool gemm_big_f32_fits(bool ta, bool tb, const GemmArgs& g);

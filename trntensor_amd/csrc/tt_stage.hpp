@@ -32,7 +32,7 @@ struct Mem16 {
 //       conflict-free stores).
 // RC k-rows are padded by 4 elements: the four lane groups of a fragment read
 // (k-rows 4 g + s) then land on disjoint LDS banks.
-template <typename T, int ROWS, bool KC, int BK>
+template <typename T, int ROWS, bool KC, int BK, int KPAD = 16 / sizeof(T), int RPAD = 4>
 struct Stage {
     static constexpr int V = Vec16<T>::n;
     static constexpr int E = ROWS * BK / kThreads;
@@ -40,8 +40,7 @@ struct Stage {
     static constexpr int TPK = BK / E;                            // KC: threads per row
     static constexpr int TPR = ROWS / V < 16 ? ROWS / V : 16;     // RC: threads per k-row
     static constexpr int NCR = KC ? NC : ROWS / (TPR * V);        // RC: pieces per k-row and thread
-    static constexpr int PAD = 16 / sizeof(T);
-    static constexpr int PITCH = KC ? (BK + PAD) : (ROWS + 4);
+    static constexpr int PITCH = KC ? (BK + KPAD) : (ROWS + RPAD);
     static constexpr int ELEMS = KC ? ROWS * PITCH : BK * PITCH;
     static_assert(BK % 16 == 0 && E % V == 0 && (KC ? BK % E == 0 : (NC % NCR == 0 && NCR >= 1)), "stage split");
     typedef typename Vec16<T>::type vec_t;
