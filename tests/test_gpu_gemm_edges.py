@@ -153,3 +153,39 @@ def test_gemm_f32_wide_tiles(hip, ta, tb, M, N, K):
     engine.gemm(ta, tb, 40, N, K, Ab, lda, sA, Bb, ldb, sB, P, N, 0, 1, 1.5, 0.5, C[0, m:], N, 0,
                 a_off=pad + (m if ta else m * lda), b_off=pad)
     assert torch.equal(P, D[0, m:])
+
+
+# fp64 sizes whose grids take 32-, 48- and 64-row direct-B tiles, ragged in the
+# columns (odd: a lane's column pair straddles the edge) and in K.
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("M,N", [(21, 60001), (17, 60030), (40, 60001), (47, 60033), (61, 60001), (150, 20003), (1000, 3001)])
+@pytest.mark.parametrize("K,with_c", [(15, True), (33, False), (64, True)])
+def test_gemm_f64_row_tiles(hip, ta, tb, M, N, K, with_c):
+    """Against float64 torch on the device, operands and D in NaN buffers, and
+    bitwise against the last columns computed in a product of 40 columns (the
+    32 x 32 tiles)."""
+    from trntensor_amd.hip import engine
+
+    dt = torch.float64
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    A = torch.randn(1, M, K, generator=g, dtype=dt, device="cuda")
+    B = torch.randn(1, K, N, generator=g, dtype=dt, device="cuda")
+    C = torch.randn(1, M, N, generator=g, dtype=dt, device="cuda") if with_c else None
+    sa, sb = A.transpose(1, 2) if ta else A, B.transpose(1, 2) if tb else B
+    lda, ldb = sa.shape[2] + 1, sb.shape[2] + 1
+    Ab, sA, _ = embed(sa, lda, 1, dt)
+    Bb, sB, _ = embed(sb, ldb, 1, dt)
+    Cb, sC, _ = embed(C, N + 1, 1, dt) if with_c else (None, 0, None)
+    Db, sD, D = embed(torch.full((1, M, N), float("nan")), N + 1, 1, dt)
+    beta = 0.5 if with_c else 0.0
+    engine.gemm(ta, tb, M, N, K, Ab, lda, sA, Bb, ldb, sB, Db, N + 1, sD, 1, 1.5, beta, Cb[1:] if with_c else None,
+                N + 1, sC, a_off=1, b_off=1, d_off=1)
+    ref = 1.5 * torch.matmul(A[0], B[0]) + (0.5 * C[0] if with_c else 0.0)
+    assert float((D[0] - ref).abs().max() / ref.abs().max()) <= TOL[dt]
+    assert int(torch.isnan(Db).sum()) == Db.numel() - M * N
+    n = N - 40
+    P = torch.empty(M, 40, dtype=dt, device="cuda")
+    Cp = C[0, :, n:].contiguous() if with_c else None
+    engine.gemm(ta, tb, M, 40, K, Ab, lda, sA, Bb, ldb, sB, P, 40, 0, 1, 1.5, beta, Cp, 40, 0, a_off=1,
+                b_off=1 + (n * ldb if tb else n))
+    assert torch.equal(P, D[0, :, n:])

@@ -19,6 +19,7 @@
 
 #include <algorithm>
 #include <type_traits>
+#include <utility>
 
 #include "tt_gemm.hpp"
 #include "tt_stage.hpp"
@@ -257,8 +258,8 @@ __global__ __launch_bounds__(kThreads) void gemm_kernel(GemmArgs g) {
 // again here rather than held through the K loop.
 // PLAIN: no C and the tile inside N (the caller checked), so every row is one
 // unconditional 16-byte store per lane.
-template <typename T, bool FULLM, bool PLAIN = false>
-__device__ __forceinline__ void directb_store(const GemmArgs& g, typename Mfma<T>::acc_t (&acc)[4][16 / sizeof(T)],
+template <typename T, bool FULLM, bool PLAIN = false, int FM = 4>
+__device__ __forceinline__ void directb_store(const GemmArgs& g, typename Mfma<T>::acc_t (&acc)[FM][16 / sizeof(T)],
                                               int64_t bat, int64_t m0, int64_t tn) {
     typedef Mfma<T> MF;
     constexpr int NB = 16 / sizeof(T);
@@ -274,7 +275,7 @@ __device__ __forceinline__ void directb_store(const GemmArgs& g, typename Mfma<T
     T* D = static_cast<T*>(g.D) + bat * g.sD;
     if constexpr (PLAIN) {
 #pragma unroll
-        for (int a = 0; a < 4; ++a)
+        for (int a = 0; a < FM; ++a)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 v16_t v;
@@ -296,10 +297,11 @@ __device__ __forceinline__ void directb_store(const GemmArgs& g, typename Mfma<T
         // against 0.1429-0.1432 ms fp32, 0.2615-0.2618 against 0.2646-0.2661
         // ms fp64; 4096^3 fp32 0.993 against 0.999 ms.
 #pragma unroll
-        for (int a2 = 0; a2 < 4; a2 += 2) {
+        for (int a2 = 0; a2 < FM; a2 += 2) {
+            constexpr int H = 2;
             v16_t cv[2][4];
 #pragma unroll
-            for (int h = 0; h < 2; ++h)
+            for (int h = 0; h < H && a2 + h < FM; ++h)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int64_t row = m0 + 16 * (a2 + h) + MF::row(lg, r);
@@ -307,7 +309,7 @@ __device__ __forceinline__ void directb_store(const GemmArgs& g, typename Mfma<T
                     cv[h][r] = *reinterpret_cast<const mem_t*>(C + (ok ? row * g.ldc + col : 0));
                 }
 #pragma unroll
-            for (int h = 0; h < 2; ++h)
+            for (int h = 0; h < H && a2 + h < FM; ++h)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int64_t row = m0 + 16 * (a2 + h) + MF::row(lg, r);
@@ -324,7 +326,7 @@ __device__ __forceinline__ void directb_store(const GemmArgs& g, typename Mfma<T
         }
     } else {
 #pragma unroll
-        for (int a = 0; a < 4; ++a)
+        for (int a = 0; a < FM; ++a)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int64_t row = m0 + 16 * a + MF::row(lg, r);
@@ -340,7 +342,7 @@ __device__ __forceinline__ void directb_store(const GemmArgs& g, typename Mfma<T
         // N - 1 (its B column was clamped): it stores those from col up.
         if (col < g.N && !colok) {
 #pragma unroll
-            for (int a = 0; a < 4; ++a)
+            for (int a = 0; a < FM; ++a)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int64_t row = m0 + 16 * a + MF::row(lg, r);
@@ -376,7 +378,7 @@ __device__ __forceinline__ void directb_store(const GemmArgs& g, typename Mfma<T
 // small-M tile: 0.877-0.883 against 0.893-0.900 ms on one box and 0.885-0.886
 // against 0.913-0.915 ms on another, alternating; M < 64 (48 x 65536 x 256,
 // four batches) measured the same.
-template <typename T, bool FULLM, bool TA, bool TB, bool NT, bool DOT>
+template <typename T, bool FULLM, bool TA, bool TB, bool NT, bool DOT, int FM = 4>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void gemm_directb_kernel(GemmArgs g) {
     typedef Mfma<T> MF;
     typedef typename MF::acc_t acc_t;
@@ -385,7 +387,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     constexpr int SPL = TB ? 16 / sizeof(T) : 1;  // MFMA steps one B load feeds (TB: k-contiguous piece)
     typedef typename VecN<T, 16 / sizeof(T)>::type v16_t;
     typedef typename Mem16<T>::type mem_t;
-    typedef Stage<T, 64, !TA, kBK> SA;  // A: a 64-row slab, [k][m] (TA) or [m][k] in LDS
+    typedef Stage<T, FM == 2 ? 32 : 64, !TA, kBK> SA;  // A: a slab of at least 16 FM rows, [k][m] (TA) or [m][k] in LDS
     __shared__ __attribute__((aligned(16))) T lds[2 * SA::ELEMS];
 
     // Tile order: the 64-row slabs of one column tile are adjacent (they
@@ -411,14 +413,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
         tn = rem / g.tiles_m;
         tm = rem - tn * g.tiles_m;
     }
-    const int64_t m0 = tm * 64;
+    const int64_t m0 = tm * (16 * FM);
     const T* A = static_cast<const T*>(g.A) + bat * g.sA;
     const int64_t nk = (g.K + kBK - 1) / kBK;
     const int64_t nfull = g.K / kBK;
 
-    acc_t acc[4][NB];
+    acc_t acc[FM][NB];
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < FM; ++a)
 #pragma unroll
         for (int b = 0; b < NB; ++b) acc[a][b] = acc_t{0, 0, 0, 0};
     if (nk > 0) {
@@ -458,7 +460,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
         // A's stage t: interior, or (K % 16 left over) the last one.
         auto aload = [&](int64_t t) __attribute__((always_inline)) { sa.template load<FULLM>(A, g.lda, m0, g.M, t * kBK); };
         auto aload_tail = [&](int64_t t) __attribute__((always_inline)) { sa.load_tail(A, g.lda, m0, g.M, t * kBK, g.K); };
-        const bool edge_m = TA && !FULLM && m0 + 64 > g.M;  // clamped pieces (uniform)
+        const bool edge_m = TA && !FULLM && m0 + (FM == 2 ? 32 : 64) > g.M;  // clamped pieces (uniform)
         auto astore = [&](int64_t t) __attribute__((always_inline)) {
             if (edge_m && t < nfull) sa.align(m0, g.M);
             sa.store(lds + (t & 1) * SA::ELEMS);
@@ -468,27 +470,27 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
         };
         // The MFMAs piece p feeds. Every accumulator still takes MFMA steps
         // 0, 1, 2, 3 in order.
-        T fa[4][SPL];
+        T fa[FM][SPL];
         auto piece = [&](const T* sbuf, int p) __attribute__((always_inline)) {
             if (!TB) {
 #pragma unroll
-                for (int a = 0; a < 4; ++a) fa[a][0] = afrag(sbuf, a, p);
+                for (int a = 0; a < FM; ++a) fa[a][0] = afrag(sbuf, a, p);
 #pragma unroll
-                for (int a = 0; a < 4; ++a)
+                for (int a = 0; a < FM; ++a)
 #pragma unroll
                     for (int b = 0; b < NB; ++b) acc[a][b] = MF::mma(fa[a][0], rb[p][b], acc[a][b]);
             } else {
                 const int h = p / NB, b = p % NB;
                 if (b == 0) {
 #pragma unroll
-                    for (int a = 0; a < 4; ++a)
+                    for (int a = 0; a < FM; ++a)
 #pragma unroll
                         for (int e = 0; e < SPL; ++e) fa[a][e] = afrag(sbuf, a, SPL * h + e);
                 }
 #pragma unroll
                 for (int e = 0; e < SPL; ++e)
 #pragma unroll
-                    for (int a = 0; a < 4; ++a) acc[a][b] = MF::mma(fa[a][e], rb[p][e], acc[a][b]);
+                    for (int a = 0; a < FM; ++a) acc[a][b] = MF::mma(fa[a][e], rb[p][e], acc[a][b]);
             }
         };
         // A wave whose columns all lie past N (in a last, partial column tile)
@@ -553,7 +555,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                 __builtin_amdgcn_sched_group_barrier(0x020, SA::NC, 0);
 #pragma unroll
                 for (int p = 0; p < 4; ++p) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 4 * NB, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x008, FM * NB, 0);
                     __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
                 }
             }
@@ -596,60 +598,69 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
         const T* E1 = static_cast<const T*>(g.E1) + bat * g.e1s[4];
         const T* E2 = g.E2 ? static_cast<const T*>(g.E2) + bat * g.e2s[4] : nullptr;
         double sum = 0.0;
-        // E2 present or not: two straight-line copies of the loop below.
-        auto dot = [&](auto has_e2) __attribute__((always_inline)) {
-            constexpr bool HE2 = decltype(has_e2)::value;
+        // E2 present or not, the tile inside the matrix or not: straight-line
+        // copies of the loop below. Row blocks outside, a block's E loads of
+        // all columns in flight together (up to 16): four round trips to
+        // memory per tile.
+        auto dot = [&](auto has_e2, auto inside) __attribute__((always_inline)) {
+            constexpr bool HE2 = decltype(has_e2)::value, IN = decltype(inside)::value;
+            // In a partial last column tile a lane that passes N computed
+            // columns N - NB .. N - 1; it owns those from col up.
+            const int64_t cw = IN ? col : min(col, g.N - NB);
+            int64_t o1n[NB], o2n[NB];
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
-                // The row parts below are formed again for every column block
-                // (the empty asm hides that they repeat): held across the
-                // blocks, they would not fit the registers of four waves per
-                // SIMD.
-                int lgb = lg;
-                asm volatile("" : "+v"(lgb));
-                // In a partial last column tile a lane that passes N computed
-                // columns N - NB .. N - 1; it owns those from col up.
-                const int64_t cw = min(col, g.N - NB) + b;
-                const bool cok = cw >= col;
-                const uint32_t cb = (uint32_t)(cok ? cw : 0);
+                const uint32_t cb = (uint32_t)(IN || cw + b >= col ? cw + b : 0);
                 const uint32_t nh = fdiv(cb, g.ndiv);
                 const uint32_t nl = cb - nh * g.ndiv.d;
-                const int64_t o1n = nh * g.e1s[2] + nl * g.e1s[3];
-                const int64_t o2n = nh * g.e2s[2] + nl * g.e2s[3];
+                o1n[b] = nh * g.e1s[2] + nl * g.e1s[3];
+                if (HE2) o2n[b] = nh * g.e2s[2] + nl * g.e2s[3];
+            }
 #pragma unroll
-                for (int a = 0; a < 4; ++a) {
-                    T e1v[4], e2v[4];
+            for (int a = 0; a < FM; ++a) {
+                T e1v[4][NB], e2v[4][NB];
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int64_t row = m0 + 16 * a + MF::row(lgb, r);
-                        const bool ok = (FULLM || row < g.M) && cok;
-                        const uint32_t rr = (uint32_t)(ok ? row : 0);
-                        const uint32_t mh = fdiv(rr, g.mdiv);
-                        const uint32_t ml = rr - mh * g.mdiv.d;
-                        e1v[r] = E1[ok ? mh * g.e1s[0] + ml * g.e1s[1] + o1n : 0];
-                        if (HE2) e2v[r] = E2[ok ? mh * g.e2s[0] + ml * g.e2s[1] + o2n : 0];
+                for (int r = 0; r < 4; ++r) {
+                    const int64_t row = m0 + 16 * a + MF::row(lg, r);
+                    const uint32_t rr = (uint32_t)(IN || row < g.M ? row : 0);
+                    const uint32_t mh = fdiv(rr, g.mdiv);
+                    const uint32_t ml = rr - mh * g.mdiv.d;
+                    const int64_t o1m = mh * g.e1s[0] + ml * g.e1s[1];
+                    const int64_t o2m = HE2 ? mh * g.e2s[0] + ml * g.e2s[1] : 0;
+#pragma unroll
+                    for (int b = 0; b < NB; ++b) {
+                        e1v[r][b] = E1[o1m + o1n[b]];
+                        if (HE2) e2v[r][b] = E2[o2m + o2n[b]];
                     }
+                }
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int64_t row = m0 + 16 * a + MF::row(lgb, r);
-                        if ((FULLM || row < g.M) && cok) {
-                            T e = e1v[r];
-                            if (HE2) e = e * e2v[r];
+                for (int r = 0; r < 4; ++r) {
+                    const int64_t row = m0 + 16 * a + MF::row(lg, r);
+#pragma unroll
+                    for (int b = 0; b < NB; ++b)
+                        if (IN || (row < g.M && cw + b >= col)) {
+                            T e = e1v[r][b];
+                            if (HE2) e = e * e2v[r][b];
                             sum += (double)(acc[a][b][r] * e);
                         }
-                    }
-                    // One block's loads in flight at a time.
-                    __builtin_amdgcn_sched_barrier(0);
                 }
+                // One block's loads in flight at a time.
+                __builtin_amdgcn_sched_barrier(0);
             }
         };
-        if (E2) dot(std::true_type{});
-        else dot(std::false_type{});
+        const bool inside = m0 + 16 * FM <= g.M && (tn + 1) * BN <= g.N;
+        if (inside) {
+            if (E2) dot(std::true_type{}, std::true_type{});
+            else dot(std::false_type{}, std::true_type{});
+        } else {
+            if (E2) dot(std::true_type{}, std::false_type{});
+            else dot(std::false_type{}, std::false_type{});
+        }
         const double tot = block256_sum(sum, red);
         if (tid == 0) g.partial[blockIdx.x] = tot;
         return;
     } else {
-        directb_store<T, FULLM>(g, acc, bat, m0, tn);
+        directb_store<T, FULLM, false, FM>(g, acc, bat, m0, tn);
     }
 }
 
@@ -1024,6 +1035,61 @@ static int launch_directb(GemmArgs& g, bool ta, bool tb, bool nt, hipStream_t st
     return check_launch("tt_gemm");
 }
 
+// fp64 direct-B tiles of 16 FM = 32 or 48 rows (rows always clamped).
+static int launch_directb_rows(GemmArgs& g, bool ta, bool tb, bool nt, int fm, hipStream_t st) {
+    g.tiles_m = (g.M + 16 * fm - 1) / (16 * fm);
+    g.tiles_n = (g.N + 127) / 128;
+    const int64_t total = g.tiles_m * g.tiles_n * g.batch;
+    if (total > 0x7fffffffLL) return set_error(TT_UNSUPPORTED, "tt_gemm: %lld tiles exceed one launch", (long long)total);
+    const dim3 grid((unsigned)total), block(kThreads);
+#define TT_ROWS_CASE(R, A_T, B_T, N_T)                 \
+    if (fm == R && ta == A_T && tb == B_T && nt == N_T) \
+        hipLaunchKernelGGL((gemm_directb_kernel<double, false, A_T, B_T, N_T, false, R>), grid, block, 0, st, g);
+#define TT_ROWS_NT(R, A_T, B_T) TT_ROWS_CASE(R, A_T, B_T, true) TT_ROWS_CASE(R, A_T, B_T, false)
+#define TT_ROWS(R) TT_ROWS_NT(R, true, true) TT_ROWS_NT(R, true, false) TT_ROWS_NT(R, false, true) TT_ROWS_NT(R, false, false)
+    TT_ROWS(2)
+    TT_ROWS(3)
+#undef TT_ROWS
+#undef TT_ROWS_NT
+#undef TT_ROWS_CASE
+    return check_launch("tt_gemm");
+}
+
+// fp64 products without the dot epilogue (all kernels bitwise equal): the tile
+// with the least estimated time of the busiest CU: its tiles times their
+// area (where a CU has several, a wave past the last column gives its share
+// back, hence columns rounded up to 32), times the kernel's cost per output,
+// times what a single direct-B tile on a CU loses because nothing covers the
+// latencies of its 16-deep stages (21 x 150 x 150 x 555 NT on fresh operands: 29
+// us on 32 x 128 tiles, 21 on 32 x 32 with 64-deep stages). us measured on 64 /
+// 48 / 32 rows x 128 columns (direct-B) / 32 x 32: 21 x 94905 x 171 TN
+// 46/38/29/40; 40 x 94905 x 171 47/40/58/67; 77 x 200000 x 300 TN
+// 274/225/227/309; 110 x 200000 x 300 275/307/284/390; 77 x 223 x 900 x 300
+// 199/198/187/246; 21 x 150 x 555 x 171 32/27/26/25; 60 x 100 x 100 x 1000 NT
+// 72/59/49/48; 3000^2 x 1000 323/289/296/350; 1400^2 x 700 56/74/57/69; 1100 x
+// 1200 x 500 41/-/-/39.5; 12 x 90 x 300 x 100 12.8/10.8/8.9/7.2.
+static int gemm_f64(GemmArgs& g, bool ta, bool tb, hipStream_t st) {
+    const bool nt = g.M <= 64 && (g.batch == 1 || g.sB != 0);  // B is read once
+    const int64_t cus = device_cus();
+    auto up = [](int64_t n, int64_t t) { return (n + t - 1) / t; };
+    const double cols = (double)(up(g.N, 32) * 32) / (double)(up(g.N, 128) * 128);
+    auto direct = [&](int64_t fm, double per_output) {
+        const int64_t rounds = up(up(g.M, 16 * fm) * up(g.N, 128) * g.batch, cus);
+        const double share = rounds == 1 ? 1.0 : rounds == 2 ? (1.0 + cols) / 2 : cols;
+        return (double)(rounds * 16 * fm * 128) * share * per_output * (rounds == 1 ? 1.6 : 1.0);
+    };
+    const int64_t sr = up(up(g.M, 32) * up(g.N, 32) * g.batch, cus);
+    const double small = (double)(sr * 32 * 32) * 1.4 * (sr <= 2 ? 1.1 : 1.0);
+    const double d4 = direct(4, 1.0), d3 = direct(3, 1.04), d2 = direct(2, 1.1);
+    // A whole 16-byte piece along a row-contiguous operand, else 32 x 32 tiles
+    // (100000 x 1 x 300 51 against 118 us on 256 x 64 LDS tiles).
+    const bool direct_ok = g.N >= 2 && (!ta || g.M >= 2);
+    if (!direct_ok || (small < d4 && small < d3 && small < d2)) return gemm_small_launch(TT_F64, ta, tb, g, st);
+    if (d2 < d4 && d2 < d3) return launch_directb_rows(g, ta, tb, nt, 2, st);
+    if (d3 < d4) return launch_directb_rows(g, ta, tb, nt, 3, st);
+    return launch_directb<double, false>(g, ta, tb, nt, st);
+}
+
 template <typename T, int BM, int BN, int FM, int FN, bool DOT, int NBUF = 2, int BK = kBK>
 static int launch_tile(GemmArgs& g, bool ta, bool tb, hipStream_t st) {
     g.tiles_m = (g.M + BM - 1) / BM;
@@ -1115,22 +1181,14 @@ static int gemm_typed(GemmArgs& g, bool ta, bool tb, hipStream_t st) {
     // (160000 x 16384 x 800, B k-contiguous) 66.2-66.4 against 67.9-68.0 ms,
     // 16900 x 900 x 450 (both extents ragged) 0.31 against 0.35 ms, the sum
     // equal to 2e-15 (another order of the per-tile sums).
-    // What is left for fp64 (N = 1 or a transposed A of one row: no whole
-    // 16-byte piece along a row-contiguous operand) runs on the 32 x 32 tiles
-    // (100000 x 1 x 300 51 against 118 us on 256 x 64 LDS tiles), with the dot epilogue
-    // on the 64 x 128 LDS tiles.
-    // Grids too small for it take the 32 x 32 tiles (tt_gemm_small.hip): fewer
-    // than 192 tiles of 64 x 128 (three quarters of the CUs). At 180 tiles
-    // (1100 x 1200 x 500) 39.5 against 40.9 us on the direct-B kernel, at 160
-    // 34.1 against 39.9, at 209 (1200 x 1300 x 500) 44.7 against 41.3, at 242
-    // (1400^2 x 700) 64 against 57.
-    if constexpr (sizeof(T) == 8) {
-        if (!DOT && ((g.M + 63) / 64) * ((g.N + 127) / 128) * g.batch < 192)
-            return gemm_small_launch(TT_F64, ta, tb, g, st);
+    // What is left for the dot (N = 1, or a transposed A of one row) runs on
+    // the 64 x 128 LDS tiles.
+    if constexpr (sizeof(T) == 8 && !DOT) {
+        return gemm_f64(g, ta, tb, st);
+    } else if constexpr (sizeof(T) == 8) {
         if (g.N >= V && (!ta || g.M >= V))
             return launch_directb<T, DOT>(g, ta, tb, g.M <= 64 && (g.batch == 1 || g.sB != 0), st);
-        if constexpr (!DOT) return gemm_small_launch(TT_F64, ta, tb, g, st);
-        else return launch_tile<T, 64, 128, 2, 4, DOT>(g, ta, tb, st);
+        return launch_tile<T, 64, 128, 2, 4, DOT>(g, ta, tb, st);
     } else if constexpr (DOT) {
         if (g.M <= 64) return launch_tile<T, 64, 128, 2, 4, DOT>(g, ta, tb, st);
         if (g.N <= 64) return launch_tile<T, 256, 64, 4, 4, DOT>(g, ta, tb, st);
@@ -1286,7 +1344,26 @@ extern "C" int tt_gemm_dot(int dtype, int transA, int transB, int64_t M, int64_t
         g.mdiv = make_fastdiv((uint32_t)mlo);
         g.ndiv = make_fastdiv((uint32_t)nlo);
         g.partial = static_cast<double*>(workspace);
-        const int rc = gemm_dot_dispatch(dtype, transA != 0, transB != 0, g, st, &nparts);
+        bool ta = transA != 0, tb = transB != 0;
+        // fp64 runs on 64 x 128 tiles: where fewer of them cover the product
+        // the other way round, X^T = op(B)^T op(A)^T is formed instead, E read
+        // with its row and column parts exchanged (16900 x 900: 1995 tiles
+        // instead of 2120).
+        if (dtype == TT_F64 && ((N + 63) / 64) * ((M + 127) / 128) < ((M + 63) / 64) * ((N + 127) / 128)) {
+            std::swap(g.A, g.B);
+            std::swap(g.M, g.N);
+            std::swap(g.lda, g.ldb);
+            std::swap(g.sA, g.sB);
+            std::swap(g.mdiv, g.ndiv);
+            for (int k = 0; k < 2; ++k) {
+                std::swap(g.e1s[k], g.e1s[k + 2]);
+                std::swap(g.e2s[k], g.e2s[k + 2]);
+            }
+            const bool t = !tb;
+            tb = !ta;
+            ta = t;
+        }
+        const int rc = gemm_dot_dispatch(dtype, ta, tb, g, st, &nparts);
         if (rc != TT_OK) return rc;
     }
     if (dtype == TT_F64)
