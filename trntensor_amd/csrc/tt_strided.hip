@@ -282,6 +282,7 @@ struct TransArgs {
     int64_t sa_u, sa_v, sd_v;
     int64_t tiles_u, tiles_v;
     Dims bat;          // sa = A strides, sb = D strides
+    bool shared;       // neighbouring tiles share cache lines (see launch_transpose)
 };
 
 template <typename T, int TS>
@@ -290,8 +291,9 @@ __global__ __launch_bounds__(256) void strided_transpose_kernel(StridedArgs g, T
     constexpr int NE = TS * TS / 256;  // elements per thread
     __shared__ T tile[TS][TS + 1];
     const int64_t per = t.tiles_u * t.tiles_v;
-    const int64_t z = blockIdx.x / per;
-    const int64_t rem = blockIdx.x - z * per;
+    const int64_t id = t.shared ? xcd_remap(blockIdx.x, gridDim.x) : blockIdx.x;
+    const int64_t z = id / per;
+    const int64_t rem = id - z * per;
     const int64_t u0 = (rem % t.tiles_u) * TS;
     const int64_t v0 = (rem / t.tiles_u) * TS;
     int64_t za, zd;
@@ -419,6 +421,18 @@ static int launch_transpose(StridedArgs& g, const int64_t* out_shape, hipStream_
     constexpr int TS = sizeof(T) == 4 ? 128 : 64;
     t.tiles_u = (t.U + TS - 1) / TS;
     t.tiles_v = (t.V + TS - 1) / TS;
+    // Rows that do not start on cache lines end in lines the next tile along
+    // the row continues. Tiles in launch order go to the XCDs in turn, so both
+    // halves of such a line then pass through different L2s: read twice, and
+    // written as two partial lines. Contiguous ranges of tiles per XCD keep
+    // them in one. us, in launch order / in ranges: 'ijk->kji' 405 x 350 x 471
+    // f64 295 / 238, f32 166 / 144; 'ijk->ikj' 270 / 218, 144 / 126; 'ijk->jki'
+    // 551 x 187 x 542 f64 227 / 183 (4.9 TB/s). Rows on whole lines keep the
+    // launch order: 'ij->ji' 16384^2 f32 418 / 469, 'ijk->ikj' 512^3 f64 358 /
+    // 377.
+    constexpr uintptr_t kLine = 128;
+    t.shared = ((reinterpret_cast<uintptr_t>(g.A) | reinterpret_cast<uintptr_t>(g.D) |
+                 (uintptr_t)(t.sa_u * (int64_t)sizeof(T)) | (uintptr_t)(t.sd_v * (int64_t)sizeof(T))) % kLine) != 0;
     t.bat.n = 0;
     int64_t nbat = 1;
     for (int k = 0; k < last; ++k) {
