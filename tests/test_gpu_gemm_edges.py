@@ -189,3 +189,35 @@ def test_gemm_f64_row_tiles(hip, ta, tb, M, N, K, with_c):
     engine.gemm(ta, tb, M, 40, K, Ab, lda, sA, Bb, ldb, sB, P, 40, 0, 1, 1.5, beta, Cp, 40, 0, a_off=1,
                 b_off=1 + (n * ldb if tb else n))
     assert torch.equal(P, D[0, :, n:])
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("M,N,K", [(33, 65, 63), (31, 129, 64), (1, 70, 40), (70, 1, 33), (7, 9, 130), (65, 63, 128),
+                                   (700, 900, 65), (2001, 1999, 33), (130, 7, 1), (520, 4100, 70)])
+def test_gemm16_unaligned_ragged(hip, dt, ta, tb, M, N, K):
+    """16-bit operands of any alignment in NaN buffers. Products and sums in
+    fp32, one rounding per output: half an ulp of the type plus the fp32 sum
+    bound K 2^-24 on sum |a b|."""
+    from trntensor_amd.hip import engine
+
+    g = torch.Generator(device="cuda").manual_seed(M * 3 + N + K)
+    for pad, with_c in ((1, True), (0, False), (3, False)):
+        A = torch.randn(1, M, K, generator=g, device="cuda").to(dt)
+        B = torch.randn(1, K, N, generator=g, device="cuda").to(dt)
+        C = torch.randn(1, M, N, generator=g, device="cuda").to(dt)
+        sa, sb = A.transpose(1, 2) if ta else A, B.transpose(1, 2) if tb else B
+        lda, ldb = sa.shape[2] + pad, sb.shape[2] + pad
+        Ab, sA, _ = embed(sa, lda, pad, dt)
+        Bb, sB, _ = embed(sb, ldb, pad, dt)
+        Cb, sC, _ = embed(C, N + pad, pad, dt)
+        Db, sD, D = embed(torch.full((1, M, N), float("nan")), N + pad, pad, dt)
+        engine.gemm(ta, tb, M, N, K, Ab, lda, sA, Bb, ldb, sB, Db, N + pad, sD, 1, 1.5, 0.5 if with_c else 0.0,
+                    Cb[pad:] if with_c else None, N + pad, sC, a_off=pad, b_off=pad, d_off=pad)
+        a, b = A[0].double(), B[0].double()
+        ref = 1.5 * (a @ b) + (0.5 * C[0].double() if with_c else 0.0)
+        mag = 1.5 * (a.abs() @ b.abs()) + (0.5 * C[0].double().abs() if with_c else 0.0)
+        ulp = 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -11
+        err = (D[0].double() - ref).abs()
+        assert bool((err <= ulp * ref.abs() + (K + 3) * 2.0 ** -24 * mag + 1e-7).all()), (pad, err.max().item())
+        assert int(torch.isnan(Db).sum()) == Db.numel() - M * N

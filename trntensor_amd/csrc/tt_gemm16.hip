@@ -4,7 +4,7 @@
 //   to the 16-bit type at the store.
 //
 // Workgroup: 256 threads = 4 wavefronts in a 2 x 2 grid over a BM x BN
-// output tile (128 x 128 or 256 x 128), each wave (BM / 2) x (BN / 2) of
+// output tile (32 x 64 to 256 x 128), each wave (BM / 2) x (BN / 2) of
 // 16 x 16 MFMA blocks with fp32 accumulators. K advances BK (64 or 32) per
 // stage through two LDS buffers (one barrier per stage), the next stage's
 // global loads held in registers during the current stage's MFMAs.
@@ -24,6 +24,8 @@
 //     16 g + 4 a + b receives element b of the blocks of lanes 16 g + 4 j + a,
 //     j = 0..3, i.e. k 8 g + 4 h .. 8 g + 4 h + 3 of row 4 a + b).
 #include <string.h>
+
+#include <algorithm>
 #include <type_traits>
 
 #include "tt_gemm.hpp"
@@ -36,6 +38,9 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
+// The same 16 bytes in memory at the element's own alignment (gfx950 serves a
+// 16-byte global access at any element address).
+typedef unsigned short u16x8_mem __attribute__((ext_vector_type(8), aligned(2)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 
 template <typename T>
@@ -75,42 +80,81 @@ struct Stage16 {
         off = (threadIdx.x % TPL) * NP * 8;
     }
 
-    // FAST: interior stage, 16-byte aligned lines: unconditional vector loads.
-    // Otherwise (a tile crossing the matrix edge, the K tail, or unaligned
-    // lines) piece by piece: a piece wholly inside is one vector load (VEC:
-    // aligned lines), one wholly outside is zero without a load, and only a
-    // piece that straddles the edge is loaded element by element from clamped
-    // addresses. (Element loads for every piece made edge tiles, and so whole
-    // ragged launches, 4-7x slower than aligned ones of the same size.)
-    template <bool FAST, bool VEC>
+    // A stage whose BK k are all in range: unconditional vector loads.
+    // INSIDE: the tile's rows are too; otherwise a KC row past the end reads
+    // the last row again and an RC piece that would pass the end starts at
+    // rows - 8 instead (rows >= 8; align() moves its elements into place):
+    // what lands in rows past the end feeds only outputs that are never
+    // stored.
+    template <bool INSIDE>
     __device__ __forceinline__ void load(const unsigned short* __restrict__ p, int64_t ld, int64_t row0, int64_t rows,
-                                         int64_t k0, int64_t kdim) {
+                                         int64_t k0) {
         int line, off;
         place(line, off);
-        if (FAST) {
-            const unsigned short* src = KC ? p + (row0 + line) * ld + k0 + off : p + (k0 + line) * ld + row0 + off;
+        if (INSIDE || KC) {
+            const int64_t row = INSIDE ? row0 + line : min(row0 + line, rows - 1);
+            const unsigned short* src = KC ? p + row * ld + k0 + off : p + (k0 + line) * ld + row0 + off;
 #pragma unroll
-            for (int c = 0; c < NP; ++c) reg[c] = *reinterpret_cast<const u16x8*>(src + 8 * c);
+            for (int c = 0; c < NP; ++c) reg[c] = *reinterpret_cast<const u16x8_mem*>(src + 8 * c);
         } else {
 #pragma unroll
             for (int c = 0; c < NP; ++c) {
-                // Piece start (gr, gk) and its extent along the contiguous direction.
-                const int64_t gr = row0 + (KC ? line : off + 8 * c);
-                const int64_t gk = k0 + (KC ? off + 8 * c : line);
-                const bool inside = KC ? (gr < rows && gk + 8 <= kdim) : (gk < kdim && gr + 8 <= rows);
-                const bool outside = gr >= rows || gk >= kdim;
-                if (VEC && inside) {
-                    reg[c] = *reinterpret_cast<const u16x8*>(KC ? p + gr * ld + gk : p + gk * ld + gr);
-                } else if (outside) {
-                    reg[c] = u16x8{0, 0, 0, 0, 0, 0, 0, 0};
-                } else {
+                const int64_t row = min(row0 + off + 8 * c, rows - 8);
+                reg[c] = *reinterpret_cast<const u16x8_mem*>(p + (k0 + line) * ld + row);
+            }
+        }
+    }
+
+    // After a clamped load of an RC operand: each piece that was started early
+    // is moved down by its overshoot.
+    __device__ __forceinline__ void align(int64_t row0, int64_t rows) {
+        if (KC) return;
+        int line, off;
+        place(line, off);
+        typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        const int64_t r = gr + (KC ? 0 : e), k = gk + (KC ? e : 0);
-                        const bool ok = r < rows && k < kdim;
-                        const unsigned short x = *(ok ? (KC ? p + r * ld + k : p + k * ld + r) : p);
-                        reg[c][e] = ok ? x : (unsigned short)0;
-                    }
+        for (int c = 0; c < NP; ++c) {
+            const int64_t over = row0 + off + 8 * c + 8 - rows;  // <= 0: not clamped; >= 8: no row inside
+            if (over <= 0 || over >= 8) continue;
+            const int sh = 16 * (int)over;
+            u64x2 x = __builtin_bit_cast(u64x2, reg[c]);
+            if (sh < 64) {
+                x[0] = (x[0] >> sh) | (x[1] << (64 - sh));
+                x[1] = x[1] >> sh;
+            } else {
+                x[0] = x[1] >> (sh - 64);
+                x[1] = 0;
+            }
+            reg[c] = __builtin_bit_cast(u16x8, x);
+        }
+    }
+
+    // The stage that passes K (zero from there), and every stage when an RC
+    // operand has fewer than 8 rows: a piece wholly inside is one vector load,
+    // one wholly outside is zero without a load, and only a piece that
+    // straddles the edge is loaded element by element from clamped addresses.
+    __device__ __forceinline__ void load_tail(const unsigned short* __restrict__ p, int64_t ld, int64_t row0,
+                                              int64_t rows, int64_t k0, int64_t kdim) {
+        int line, off;
+        place(line, off);
+#pragma unroll
+        for (int c = 0; c < NP; ++c) {
+            // Piece start (gr, gk) and its extent along the contiguous direction.
+            const int64_t gr = row0 + (KC ? line : off + 8 * c);
+            const int64_t gk = k0 + (KC ? off + 8 * c : line);
+            const bool inside = KC ? (gr < rows && gk + 8 <= kdim) : (gk < kdim && gr + 8 <= rows);
+            const bool outside = gr >= rows || gk >= kdim;
+            if (inside) {
+                reg[c] = *reinterpret_cast<const u16x8_mem*>(KC ? p + gr * ld + gk : p + gk * ld + gr);
+            } else if (outside) {
+                reg[c] = u16x8{0, 0, 0, 0, 0, 0, 0, 0};
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const int64_t r = gr + (KC ? 0 : e), k = gk + (KC ? e : 0);
+                    const bool ok = r < rows && k < kdim;
+                    const unsigned short x = *(ok ? (KC ? p + r * ld + k : p + k * ld + r) : p);
+                    reg[c][e] = ok ? x : (unsigned short)0;
                 }
             }
         }
@@ -146,7 +190,8 @@ __device__ __forceinline__ unsigned short from_f32(float x) {
     return __builtin_bit_cast(unsigned short, (T)x);
 }
 
-template <typename T, bool TA, bool TB, bool VEC, int BM, int BN, int BK>
+// FULL: M and N are multiples of the tile (no row or column clamping).
+template <typename T, bool TA, bool TB, bool FULL, int BM, int BN, int BK>
 __global__ __launch_bounds__(256) void gemm16_kernel(GemmArgs g) {
     // A rows are m: k-contiguous unless transposed. B rows are n: k-contiguous iff transposed.
     typedef Stage16<!TA, BM, BK> SA;
@@ -188,11 +233,22 @@ __global__ __launch_bounds__(256) void gemm16_kernel(GemmArgs g) {
     SA sa;
     SB sb;
     const int64_t nk = (g.K + BK - 1) / BK;
-    const int64_t nfull = (VEC && m0 + BM <= g.M && n0 + BN <= g.N) ? g.K / BK : 0;
-    auto load = [&](int64_t k0, auto fast) {
-        constexpr bool F = decltype(fast)::value;
-        sa.template load<F, VEC>(A, g.lda, m0, g.M, k0, g.K);
-        sb.template load<F, VEC>(B, g.ldb, n0, g.N, k0, g.K);
+    // Stages 0 .. nfull-1 have all their k in range (a row-contiguous operand
+    // with fewer rows than one vector takes the guarded loads throughout).
+    const int64_t nfull = (!TA || g.M >= 8) && (TB || g.N >= 8) ? g.K / BK : 0;
+    auto load = [&](int64_t k0) __attribute__((always_inline)) {
+        sa.template load<FULL>(A, g.lda, m0, g.M, k0);
+        sb.template load<FULL>(B, g.ldb, n0, g.N, k0);
+    };
+    auto load_tail = [&](int64_t k0) __attribute__((always_inline)) {
+        sa.load_tail(A, g.lda, m0, g.M, k0, g.K);
+        sb.load_tail(B, g.ldb, n0, g.N, k0, g.K);
+    };
+    // Pieces that were clamped at the matrix edge (uniform: edge tiles only).
+    const bool edge_m = TA && !FULL && m0 + BM > g.M, edge_n = !TB && !FULL && n0 + BN > g.N;
+    auto align = [&]() __attribute__((always_inline)) {
+        if (edge_m) sa.align(m0, g.M);
+        if (edge_n) sb.align(n0, g.N);
     };
     auto compute = [&](int buf) {
         const unsigned short* a = bufA(buf);
@@ -212,16 +268,21 @@ __global__ __launch_bounds__(256) void gemm16_kernel(GemmArgs g) {
     };
     int64_t kt = 0;
     if (nk > 0) {
-        if (nfull > 0) load(0, std::true_type{});
-        else load(0, std::false_type{});
+        if (nfull > 0) {
+            load(0);
+            align();
+        } else {
+            load_tail(0);
+        }
         sa.store(bufA(0));
         sb.store(bufB(0));
     }
     __syncthreads();
     for (; kt + 1 < nfull; ++kt) {
-        load((kt + 1) * BK, std::true_type{});
+        load((kt + 1) * BK);
         compute(kt & 1);
         __builtin_amdgcn_sched_barrier(0);
+        align();
         sa.store(bufA((kt & 1) ^ 1));
         sb.store(bufB((kt & 1) ^ 1));
         __syncthreads();
@@ -229,7 +290,7 @@ __global__ __launch_bounds__(256) void gemm16_kernel(GemmArgs g) {
     // Buffer kt & 1 holds stage kt; the remaining stages load one ahead.
     for (; kt < nk; ++kt) {
         const bool more = kt + 1 < nk;
-        if (more) load((kt + 1) * BK, std::false_type{});
+        if (more) load_tail((kt + 1) * BK);
         compute(kt & 1);
         __builtin_amdgcn_sched_barrier(0);
         if (more) {
@@ -250,8 +311,6 @@ __global__ __launch_bounds__(256) void gemm16_kernel(GemmArgs g) {
     constexpr int SP = WN + 4;  // slab pitch in floats (16-byte multiple)
     static_assert(4 * 16 * SP * sizeof(float) <= sizeof(lds), "epilogue slabs fit in the stage buffers");
     float* slab = reinterpret_cast<float*>(lds) + wave * 16 * SP;
-    auto a16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-    const bool vout = a16(D) && g.ldd % 8 == 0 && (!C || (a16(C) && g.ldc % 8 == 0));
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
         // This slab's C chunks are loaded before any of its stores (and before the
@@ -266,7 +325,7 @@ __global__ __launch_bounds__(256) void gemm16_kernel(GemmArgs g) {
             const int64_t row = m0 + wm0 + 16 * i + rr;
             const int64_t col = n0 + wn0 + 8 * cb;
             cc[h] = u16x8{0, 0, 0, 0, 0, 0, 0, 0};
-            if (C && vout && row < g.M && col + 8 <= g.N) cc[h] = *reinterpret_cast<const u16x8*>(C + row * g.ldc + col);
+            if (C && row < g.M && col + 8 <= g.N) cc[h] = *reinterpret_cast<const u16x8_mem*>(C + row * g.ldc + col);
         }
 #pragma unroll
         for (int j = 0; j < FN; ++j)
@@ -287,7 +346,7 @@ __global__ __launch_bounds__(256) void gemm16_kernel(GemmArgs g) {
             const f32x4 hi = *reinterpret_cast<const f32x4*>(slab + rr * SP + 8 * cb + 4);
             float x[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
             if (row < g.M) {
-                if (vout && col + 8 <= g.N) {
+                if (col + 8 <= g.N) {
                     if (C) {
 #pragma unroll
                         for (int e = 0; e < 8; ++e) x[e] = x[e] + beta * to_f32<T>(cc[h][e]);
@@ -295,7 +354,7 @@ __global__ __launch_bounds__(256) void gemm16_kernel(GemmArgs g) {
                     u16x8 d;
 #pragma unroll
                     for (int e = 0; e < 8; ++e) d[e] = from_f32<T>(x[e]);
-                    *reinterpret_cast<u16x8*>(D + row * g.ldd + col) = d;
+                    *reinterpret_cast<u16x8_mem*>(D + row * g.ldd + col) = d;
                 } else {
 #pragma unroll
                     for (int e = 0; e < 8; ++e)
@@ -312,15 +371,16 @@ __global__ __launch_bounds__(256) void gemm16_kernel(GemmArgs g) {
 }
 
 template <typename T, int BM, int BN, int BK>
-int launch16(bool ta, bool tb, bool vec, GemmArgs& g, hipStream_t st) {
+int launch16(bool ta, bool tb, GemmArgs& g, hipStream_t st) {
     g.tiles_m = (g.M + BM - 1) / BM;
     g.tiles_n = (g.N + BN - 1) / BN;
     const int64_t total = g.tiles_m * g.tiles_n * g.batch;
     if (total > 0x7fffffffLL) return set_error(TT_UNSUPPORTED, "tt_gemm: %lld tiles exceed one launch", (long long)total);
+    const bool full = g.M % BM == 0 && g.N % BN == 0;
     const dim3 grid((unsigned)total), block(256);
-#define TT_GEMM16_CASE(TA, TB, VC)           \
-    if (ta == TA && tb == TB && vec == VC) \
-        hipLaunchKernelGGL((gemm16_kernel<T, TA, TB, VC, BM, BN, BK>), grid, block, 0, st, g);
+#define TT_GEMM16_CASE(TA, TB, F)           \
+    if (ta == TA && tb == TB && full == F) \
+        hipLaunchKernelGGL((gemm16_kernel<T, TA, TB, F, BM, BN, BK>), grid, block, 0, st, g);
     TT_GEMM16_CASE(false, false, false)
     TT_GEMM16_CASE(false, false, true)
     TT_GEMM16_CASE(false, true, false)
@@ -333,22 +393,43 @@ int launch16(bool ta, bool tb, bool vec, GemmArgs& g, hipStream_t st) {
     return check_launch("tt_gemm (16-bit)");
 }
 
+int64_t up(int64_t n, int64_t t) { return (n + t - 1) / t; }
+
+// Estimated time of the busiest CU (arbitrary units): its bm x bn tiles times
+// their area, times the kernel's cost per output where every CU has many
+// tiles, times what a single tile on a CU loses because nothing covers its
+// latencies.
+double cost16(const GemmArgs& g, int64_t bm, int64_t bn, double per_output, double one) {
+    const int64_t rounds = up(up(g.M, bm) * up(g.N, bn) * g.batch, device_cus());
+    return (double)(rounds * bm * bn) * per_output * (rounds == 1 ? one : 1.0);
+}
+
+// The register-staged kernel's tile: 0: 128 x 128, 1: 64 x 64, 2: 32 x 64. us
+// measured (bf16): 787 x 423 x 3415 106/51/40 (336 with element-wise loads of
+// the odd rows on 128 x 128), 4332 x 1643 x 1352 TT 48/59/86 (241), 2001 x 3003 x
+// 1001 49/45/58 (172), 684 x 5650 x 287 22/13/16 (53), 1236 x 2965 x 167 TT
+// 16/12/14 (32), 1672 x 194 x 241 TT 11.6/6.6/5.8 (27), 1024^3 17.6/10.8/10.7,
+// 1591 x 225 x 5665 219/80/63 (527). 64 x 128 tiles were within 5% of the best of
+// these or behind it, 128-deep stages 10% faster on 32 x 64 with B
+// k-contiguous and few tiles, up to 1.6 times slower elsewhere.
+double staged_cost(const GemmArgs& g, int* tile) {
+    const double c[3] = {cost16(g, 128, 128, 1.0, 1.5), cost16(g, 64, 64, 1.3, 1.5), cost16(g, 32, 64, 1.8, 1.5)};
+    *tile = (int)(std::min_element(c, c + 3) - c);
+    return c[*tile];
+}
+
 // Register-staged kernel (any shape, alignment and K).
 template <typename T>
 int gemm16_staged(bool ta, bool tb, GemmArgs& g, hipStream_t st) {
-    auto ok16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-    bool vec = ok16(g.A) && ok16(g.B) && g.lda % 8 == 0 && g.ldb % 8 == 0;
-    if (g.batch > 1) vec = vec && g.sA % 8 == 0 && g.sB % 8 == 0;
-    // Measured at 4096^3 (bf16): with A row-contiguous (transposed), 256 x 128
-    // tiles of depth 32 run at 934-939 TFLOP/s against 840-862 for 128 x 128 x 64;
-    // with A k-contiguous the 128 x 128 x 64 tile is the faster (857-872 against
-    // 827-871). 128 x 256 x 32 and 128 x 128 x 32 tiles measured 802-922 and
-    // 710-868; 128 x 256 x 64 (one workgroup per CU) 500. On smaller grids the
-    // 256 x 128 tile leaves CUs idle: 8 x 384 x 1024^2 41 against 282-288,
-    // 2048^3 252 against 394-399, 4096 x 256 x 4096 68 against 113-115.
-    if (ta && ((g.M + 255) / 256) * ((g.N + 127) / 128) * g.batch >= 512)
-        return launch16<T, 256, 128, 32>(ta, tb, vec, g, st);
-    return launch16<T, 128, 128, 64>(ta, tb, vec, g, st);
+    // Many tiles with A row-contiguous: 256 x 128 tiles of depth 32 (4096^3,
+    // bf16: 934-939 against 840-862 TFLOP/s on 128 x 128 x 64; 4095^3 TN 202
+    // against 329 us).
+    if (ta && up(g.M, 256) * up(g.N, 128) * g.batch >= 512) return launch16<T, 256, 128, 32>(ta, tb, g, st);
+    int tile;
+    staged_cost(g, &tile);
+    if (tile == 2) return launch16<T, 32, 64, 64>(ta, tb, g, st);
+    if (tile == 1) return launch16<T, 64, 64, 64>(ta, tb, g, st);
+    return launch16<T, 128, 128, 64>(ta, tb, g, st);
 }
 
 template <typename T>
@@ -363,27 +444,22 @@ int gemm16_typed(bool ta, bool tb, GemmArgs& g, hipStream_t st) {
     // 398-403 against 400-401, TT 419 against 392-396; 64 x 512^3: 588-669
     // against 508-562).
     const int64_t kmin = 256;
-    // It also needs a full grid, and the ragged strips run as separate,
-    // serial launches: against the register-staged kernel alone it lost with
-    // 96-128 whole tiles (8 x 384 x 1024^2: 228-241 against 282-298 TFLOP/s;
-    // 2048^3: 359-387 against 394-411), tied at 192-256 (16 x 512 x 1024^2:
-    // 572-602 against 574-612) and won at 512 (4096^3 NN: 1104 against 850);
-    // with strips of a tenth of the outputs (2000 x 3000 x 320) it ran at
-    // 31-43 against 71-74. Its 128 x 128 tile (three workgroups per CU) takes
-    // the grids too small for 128 x 256 and beats the register-staged kernel
-    // on the same grid from 64 tiles (2048^3: 512-544 against 397-406;
-    // 8 x 384 x 1024^2: 320-335 against 293-302; 4096 x 256 x 4096: 151-162
-    // against 113-117, NT 112 against 113); with strips of 5.8% of the
-    // outputs (2000 x 3000 x 320) it lost again, 42-48 against 71-75, so
-    // strips are limited to 1/64.
+    // The ragged strips run as separate, serial launches, so they are limited
+    // to 1/64 of the outputs (2000 x 3000 x 320, 5.8% in strips: 42-48 against
+    // 71-75 TFLOP/s on the register-staged kernel alone). On its 128 x 256 or 128
+    // x 128 tiles the kernel costs 0.7 of the staged 128 x 128 tile's time per
+    // output (4096^3 NN 120 against 172 us, 2048^3 33 against 44), so smaller
+    // staged tiles take the grids that leave its CUs idle (2048^3 40 us on 64 x
+    // 64; 1024^3 17.7 against 10.7 us).
     int bm_, bn_;
     gemm16_dma_tile(ta, tb, g.M, g.N, g.K, g.batch, bm_, bn_);
     const int64_t bm = bm_, bn = bn_;
     const int64_t Mi = g.M & ~(bm - 1), Ni = g.N & ~(bn - 1);
-    const int64_t tiles = (Mi / bm) * (Ni / bn) * g.batch;
     const bool small_strips = (g.M - Mi) * g.N + Mi * (g.N - Ni) <= g.M * g.N / 64;
-    if (!vec || g.M < bm || g.N < bn || g.K < kmin || g.K % 32 != 0 || tiles < 64 || !small_strips)
+    if (!vec || g.M < bm || g.N < bn || g.K < kmin || g.K % 32 != 0 || !small_strips)
         return gemm16_staged<T>(ta, tb, g, st);
+    int tile;
+    if (cost16(g, bm, bn, 0.7, 1.5) > staged_cost(g, &tile)) return gemm16_staged<T>(ta, tb, g, st);
     // Whole bm x bn tiles by the direct-load kernel; the ragged row and
     // column strips (if any) by the register-staged kernel on sub-matrices.
     const unsigned short* A = static_cast<const unsigned short*>(g.A);
