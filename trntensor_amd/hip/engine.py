@@ -182,13 +182,18 @@ def strided_contract(
     A/B's first element (``data_ptr()``) plus a_off/b_off. Launches are split so every index
     range stays below 2^31.
     """
-    lib = _lib.load()
+    if D.numel() == 0:
+        return
+    code = dtype_code(D.dtype)
+    key = (code, tuple(out_dims), tuple(red_dims))
+    spec = _STRIDED.get(key)
+    if spec is not None:
+        _launch_strided(spec, code, A, B, D, alpha, beta, C, a_off, b_off)
+        return
     out_dims = _merge_dims(out_dims)
     red_dims = _merge_dims(red_dims)
     n_out = _numel(d[0] for d in out_dims)
     n_red = _numel(d[0] for d in red_dims)
-    if n_out == 0:
-        return
     if len(out_dims) > _lib.TT_MAX_DIMS or len(red_dims) > _lib.TT_MAX_DIMS:
         raise NotImplementedError("contraction with more than 8 independent strided dimensions")
 
@@ -242,39 +247,36 @@ def strided_contract(
             first = False
         return
 
-    code = dtype_code(D.dtype)
+    oshape, rshape = _lib.i64_array(d[0] for d in out_dims), _lib.i64_array(d[0] for d in red_dims)
+    spec = (
+        len(out_dims), oshape, _lib.i64_array(d[1] for d in out_dims), _lib.i64_array(d[2] for d in out_dims),
+        len(red_dims), rshape, _lib.i64_array(d[1] for d in red_dims), _lib.i64_array(d[2] for d in red_dims),
+        _lib.load().tt_strided_contract_workspace_bytes(code, len(out_dims), oshape, len(red_dims), rshape),
+    )
+    if len(_STRIDED) >= _STRIDED_MAX:
+        _STRIDED.clear()
+    _STRIDED[key] = spec
+    _launch_strided(spec, code, A, B, D, alpha, beta, C, a_off, b_off)
+
+
+# Merged dimensions, their ctypes arrays and the workspace size of launches
+# that need no splitting, keyed by (dtype code, output dims, reduction dims);
+# bounded. Read-only once built: the library copies them per launch.
+_STRIDED: dict[tuple, tuple] = {}
+_STRIDED_MAX = 1024
+
+
+def _launch_strided(spec, code, A, B, D, alpha, beta, C, a_off, b_off) -> None:
+    no, oshape, oa, ob, nr, rshape, ra, rb, wsb = spec
     es = D.element_size()
-    oshape = _lib.i64_array(d[0] for d in out_dims)
-    oa = _lib.i64_array(d[1] for d in out_dims)
-    ob = _lib.i64_array(d[2] for d in out_dims)
-    rshape = _lib.i64_array(d[0] for d in red_dims)
-    ra = _lib.i64_array(d[1] for d in red_dims)
-    rb = _lib.i64_array(d[2] for d in red_dims)
-    wsb = lib.tt_strided_contract_workspace_bytes(code, len(out_dims), oshape, len(red_dims), rshape)
     ws = _workspace(wsb, D.device)
-    a_ptr = A.data_ptr() + a_off * es
-    b_ptr = None if B is None else B.data_ptr() + b_off * es
-    st = lib.tt_strided_contract(
-        code,
-        len(out_dims),
-        oshape,
-        oa,
-        ob,
-        len(red_dims),
-        rshape,
-        ra,
-        rb,
-        a_ptr,
-        b_ptr,
-        float(alpha),
-        float(beta),
-        _ptr(C),
-        _ptr(D),
-        _ptr(ws),
-        wsb,
+    st = _lib.load().tt_strided_contract(
+        code, no, oshape, oa, ob, nr, rshape, ra, rb, A.data_ptr() + a_off * es,
+        None if B is None else B.data_ptr() + b_off * es, float(alpha), float(beta), _ptr(C), _ptr(D), _ptr(ws), wsb,
         _stream_ptr(D.device),
     )
-    _lib.check(st, "tt_strided_contract")
+    if st:
+        _lib.check(st, "tt_strided_contract")
 
 
 def pack(op: Operand, order: list[str]) -> torch.Tensor:
