@@ -221,3 +221,26 @@ def test_gemm16_unaligned_ragged(hip, dt, ta, tb, M, N, K):
         err = (D[0].double() - ref).abs()
         assert bool((err <= ulp * ref.abs() + (K + 3) * 2.0 ** -24 * mag + 1e-7).all()), (pad, err.max().item())
         assert int(torch.isnan(Db).sum()) == Db.numel() - M * N
+
+
+@pytest.mark.parametrize("kind,batch,M,N", [("f32", 2**23 + 5, 33, 1), ("f64", 2**23 + 5, 33, 1),
+                                            ("dd", 2**23 + 5, 17, 1), ("bf16", 2**23 + 5, 33, 1),
+                                            ("f64", 1, 2**29 + 40, 1), ("f32", 1, 1, 2**29 + 40)])
+def test_gemm_more_tiles_than_a_grid(hip, kind, batch, M, N):
+    """2^24 small tiles and more do not fit one launch: larger tiles or
+    several launches take them. K = 1, so every output is one rounded product
+    (the double-double sum included) and equals torch's."""
+    import contextlib
+
+    from trntensor_amd.hip import engine
+
+    dt = {"f32": torch.float32, "bf16": torch.bfloat16}.get(kind, torch.float64)
+    g = torch.Generator(device="cuda").manual_seed(batch + M)
+    A = torch.randn(batch, M, 1, generator=g, dtype=torch.float32, device="cuda").to(dt)
+    B = torch.randn(batch, 1, N, generator=g, dtype=torch.float32, device="cuda").to(dt)
+    D = torch.full((batch, M, N), float("nan"), dtype=dt, device="cuda")
+    with engine.accumulation("dd") if kind == "dd" else contextlib.nullcontext():
+        # A one-row matrix is passed as its transpose (leading dimension M = 1).
+        ta = M == 1
+        engine.gemm(ta, False, M, N, 1, A, M if ta else 1, M, B, N, N, D, N, M * N, batch, 1.0, 0.0, None, 0, 0)
+    assert torch.equal(D, A * B)

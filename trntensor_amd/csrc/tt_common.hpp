@@ -193,6 +193,10 @@ __device__ __forceinline__ uint32_t fdiv(uint32_t n, const FastDiv& f) {
     return (__umulhi(n, f.m) + n) >> f.s;
 }
 
+// Workgroups of 256 threads that one launch may have: HIP counts a grid's
+// threads in 32 bits, and a launch of more runs too few without an error.
+constexpr int64_t kMaxGrid = 0xffffffffLL / 256;
+
 // ---------------------------------------------------------------------------
 // Status plumbing
 // ---------------------------------------------------------------------------

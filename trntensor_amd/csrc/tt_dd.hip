@@ -142,6 +142,12 @@ int launch_dd(bool ta, bool tb, GemmArgs& g, hipStream_t st) {
     const int64_t total = g.tiles_m * g.tiles_n * g.batch;
     if (total > 0x7fffffffLL)
         return set_error(TT_UNSUPPORTED, "tt_gemm: %lld tiles exceed one launch", (long long)total);
+    if (total > kMaxGrid) {
+        GemmArgs lo = g, hi = g;
+        split_gemm(sizeof(double), ta, tb, 64, lo, hi);
+        const int rc = launch_dd<RM, RN>(ta, tb, lo, st);
+        return rc == TT_OK ? launch_dd<RM, RN>(ta, tb, hi, st) : rc;
+    }
     const dim3 grid((unsigned)total), block(256);
     if (!ta && !tb) hipLaunchKernelGGL((gemm_dd_kernel<false, false, RM, RN>), grid, block, 0, st, g);
     if (!ta && tb) hipLaunchKernelGGL((gemm_dd_kernel<false, true, RM, RN>), grid, block, 0, st, g);

@@ -1074,7 +1074,9 @@ static int gemm_f64(GemmArgs& g, bool ta, bool tb, hipStream_t st) {
     auto up = [](int64_t n, int64_t t) { return (n + t - 1) / t; };
     const double cols = (double)(up(g.N, 32) * 32) / (double)(up(g.N, 128) * 128);
     auto direct = [&](int64_t fm, double per_output) {
-        const int64_t rounds = up(up(g.M, 16 * fm) * up(g.N, 128) * g.batch, cus);
+        const int64_t n = up(g.M, 16 * fm) * up(g.N, 128) * g.batch;
+        if (n > kMaxGrid) return 1e300;  // not one launch; the 32 x 32 tiles take several
+        const int64_t rounds = up(n, cus);
         const double share = rounds == 1 ? 1.0 : rounds == 2 ? (1.0 + cols) / 2 : cols;
         return (double)(rounds * 16 * fm * 128) * share * per_output * (rounds == 1 ? 1.6 : 1.0);
     };
@@ -1142,13 +1144,14 @@ static int gemm_f32(GemmArgs& g, bool ta, bool tb, hipStream_t st) {
     // 150 x 2000 x 3000 -/186/105/86/52; 4000^2 x 1000 -/260/268/285/311; 64 x
     // 786432 x 512 TN 452/787/470/535/623; 80 x 200000 x 300 TN
     // -/156/150/170/160.
+    const double never = 1e300;
     auto cost = [&](int64_t bm, int64_t bn, double per_output, double one, double two) {
         const int64_t n = ((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn) * g.batch;
+        if (n > kMaxGrid && bm > 32) return never;  // not one launch; the 32 x 32 tiles take several
         const int64_t rounds = (n + cus - 1) / cus;
         return (double)(rounds * bm * bn) * per_output * (rounds == 1 ? one : rounds == 2 ? two : 1.0);
     };
     const bool rows_ok = !ta || g.M >= 4, cols_ok = tb || g.N >= 4;  // a 16-byte piece along a row-contiguous operand
-    const double never = 1e300;
     const double direct = rows_ok && !tb && g.N % 256 == 0 ? cost(64, 256, 0.97, 1.1, 1.0) : never;
     const double tall = rows_ok && cols_ok && g.K > 0 ? cost(128, 128, 1.0, 1.05, 1.0) : never;
     const double mid = rows_ok && cols_ok && g.K > 0 ? cost(64, 128, 1.04, 1.05, 1.0) : never;

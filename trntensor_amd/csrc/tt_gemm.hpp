@@ -28,6 +28,33 @@ struct GemmArgs {
     double* partial;
 };
 
+// A product with more tiles than a launch may have workgroups runs as two,
+// lo and hi (both copies of it): halves of the batch, or of the longer side,
+// at a multiple of `unit` rows or columns.
+inline void split_gemm(size_t elem, bool ta, bool tb, int64_t unit, GemmArgs& lo, GemmArgs& hi) {
+    const GemmArgs g = lo;
+    const int64_t tm = (g.M + unit - 1) / unit, tn = (g.N + unit - 1) / unit;
+    int64_t a = 0, b = 0, c = 0, d = 0;
+    if (g.batch > 1) {
+        lo.batch = g.batch / 2;
+        hi.batch = g.batch - lo.batch;
+        a = lo.batch * g.sA, b = lo.batch * g.sB, c = lo.batch * g.sC, d = lo.batch * g.sD;
+    } else if (tm >= tn) {
+        lo.M = tm / 2 * unit;
+        hi.M = g.M - lo.M;
+        a = ta ? lo.M : lo.M * g.lda, c = lo.M * g.ldc, d = lo.M * g.ldd;
+    } else {
+        lo.N = tn / 2 * unit;
+        hi.N = g.N - lo.N;
+        b = tb ? lo.N * g.ldb : lo.N, c = lo.N, d = lo.N;
+    }
+    auto at = [&](const void* p, int64_t n) { return p ? static_cast<const char*>(p) + n * (int64_t)elem : nullptr; };
+    hi.A = at(g.A, a);
+    hi.B = at(g.B, b);
+    hi.C = at(g.C, c);
+    hi.D = static_cast<char*>(g.D) + d * (int64_t)elem;
+}
+
 // Compute units of the current device (cached per device).
 int device_cus();
 // tt_gemm after argument checks (store epilogue).

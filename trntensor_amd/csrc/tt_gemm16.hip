@@ -376,6 +376,12 @@ int launch16(bool ta, bool tb, GemmArgs& g, hipStream_t st) {
     g.tiles_n = (g.N + BN - 1) / BN;
     const int64_t total = g.tiles_m * g.tiles_n * g.batch;
     if (total > 0x7fffffffLL) return set_error(TT_UNSUPPORTED, "tt_gemm: %lld tiles exceed one launch", (long long)total);
+    if (total > kMaxGrid) {
+        GemmArgs lo = g, hi = g;
+        split_gemm(2, ta, tb, 256, lo, hi);
+        const int rc = launch16<T, BM, BN, BK>(ta, tb, lo, st);
+        return rc == TT_OK ? launch16<T, BM, BN, BK>(ta, tb, hi, st) : rc;
+    }
     const bool full = g.M % BM == 0 && g.N % BN == 0;
     const dim3 grid((unsigned)total), block(256);
 #define TT_GEMM16_CASE(TA, TB, F)           \

@@ -164,6 +164,12 @@ int launch(bool ta, bool tb, GemmArgs& g, hipStream_t st) {
     g.tiles_n = (g.N + kSmall - 1) / kSmall;
     const int64_t total = g.tiles_m * g.tiles_n * g.batch;
     if (total > 0x7fffffffLL) return set_error(TT_UNSUPPORTED, "tt_gemm: %lld tiles exceed one launch", (long long)total);
+    if (total > kMaxGrid) {
+        GemmArgs lo = g, hi = g;
+        split_gemm(sizeof(T), ta, tb, kSmall, lo, hi);
+        const int rc = launch<T>(ta, tb, lo, st);
+        return rc == TT_OK ? launch<T>(ta, tb, hi, st) : rc;
+    }
     // One 128-deep fp32 stage holds K <= 128 (fp64: 64, as any stage).
     const bool deep = sizeof(T) == 4 && g.K > 64 && g.K <= 128;
     const bool full = g.M % kSmall == 0 && g.N % kSmall == 0;
