@@ -26,3 +26,12 @@ def test_permute_edges(hip, dt, sub, shape):
         c = torch.randn([shape[k] for k in order], generator=g, dtype=torch.float64).to(dt)
         got = tt.einsum(sub, v, alpha=2.0, beta=0.5, out=c.cuda())
         assert torch.equal(got.cpu(), 2.0 * x.permute(order) + 0.5 * c)
+
+
+def test_permute_more_tiles_than_a_grid(hip):
+    """One small transpose per batch entry, 2^24 and more of them: their tiles
+    do not fit one launch."""
+    import trntensor_amd as tt
+
+    x = torch.arange(6 * (2**24 + 5), dtype=torch.float32, device="cuda").view(2**24 + 5, 2, 3)
+    assert torch.equal(tt.einsum("aij->aji", x), x.transpose(1, 2).contiguous())

@@ -22,6 +22,7 @@
 // (trntensor/quantum.py:97-99): denominator ((e_i + e_j) - e_a) - e_b with a
 // the row index, term (T * (2T - T^T)) / denominator with IEEE division, in
 // the input dtype; the energy is accumulated in double.
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
@@ -732,7 +733,6 @@ static int mp2_typed(int64_t nocc, int64_t nvir, int64_t naux, const void* B, co
     g.npq = (int64_t)g.nblk * (g.nblk + 1) / 2;
     g.group = mp2_pair_group(nocc);
     g.first = first;
-    g.ntasks = count;
     double* w = static_cast<double*>(ws);
     if (det) {
         g.partial = w;
@@ -743,14 +743,18 @@ static int mp2_typed(int64_t nocc, int64_t nvir, int64_t naux, const void* B, co
         hipLaunchKernelGGL(zero_double_kernel, dim3(1), dim3(64), 0, st, w);
     }
     constexpr int BK = kMp2StageK;
-    if (g.ntasks > 0) {
-        if (nvir % kMp2Tile >= 1 && nvir % kMp2Tile <= 32)
-            hipLaunchKernelGGL((mp2_energy_kernel<T, BK, true>), dim3((unsigned)g.ntasks), dim3(kMp2Threads), 0, st, g);
-        else
-            hipLaunchKernelGGL((mp2_energy_kernel<T, BK, false>), dim3((unsigned)g.ntasks), dim3(kMp2Threads), 0, st, g);
+    const bool tail = nvir % kMp2Tile >= 1 && nvir % kMp2Tile <= 32;
+    for (int64_t done = 0; done < count; done += g.ntasks) {
+        Mp2Args l = g;
+        l.first = first + done;
+        l.ntasks = g.ntasks = std::min(count - done, kMaxGrid);
+        if (det) l.partial = w + done;
+        const dim3 grid((unsigned)l.ntasks), block(kMp2Threads);
+        if (tail) hipLaunchKernelGGL((mp2_energy_kernel<T, BK, true>), grid, block, 0, st, l);
+        else hipLaunchKernelGGL((mp2_energy_kernel<T, BK, false>), grid, block, 0, st, l);
     }
     hipLaunchKernelGGL(mp2_finalize_kernel<T>, dim3(1), dim3(256), 0, st, (const double*)w,
-                       det ? g.ntasks : (int64_t)1, static_cast<T*>(out));
+                       det ? count : (int64_t)1, static_cast<T*>(out));
     return check_launch("tt_mp2_energy");
 }
 

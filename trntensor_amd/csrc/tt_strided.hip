@@ -445,6 +445,10 @@ static int launch_transpose(StridedArgs& g, const int64_t* out_shape, hipStream_
     }
     const int64_t blocks = t.tiles_u * t.tiles_v * nbat;
     if (blocks > 0x7fffffffLL) return set_error(TT_UNSUPPORTED, "tt_strided_contract: %lld tiles", (long long)blocks);
+    if (blocks > kMaxGrid) {  // a grid-stride loop over the outputs instead
+        hipLaunchKernelGGL((strided_per_output_kernel<T, false>), dim3(1 << 20), dim3(256), 0, st, g);
+        return TT_OK;
+    }
     hipLaunchKernelGGL((strided_transpose_kernel<T, TS>), dim3((unsigned)blocks), dim3(256), 0, st, g, t);
     return TT_OK;
 }
