@@ -244,3 +244,22 @@ def test_gemm_more_tiles_than_a_grid(hip, kind, batch, M, N):
         ta = M == 1
         engine.gemm(ta, False, M, N, 1, A, M if ta else 1, M, B, N, N, D, N, M * N, batch, 1.0, 0.0, None, 0, 0)
     assert torch.equal(D, A * B)
+
+
+@pytest.mark.parametrize("dt", [torch.float64, torch.float32])
+@pytest.mark.parametrize("batch,M,N", [(2**24 + 5, 1, 1), (2**24 + 5, 1, 2), (1, 2**20 + 1, 2**18 + 1)])
+def test_gemm_dot_more_tiles_than_a_grid(hip, dt, batch, M, N):
+    """A dot of 2^24 tiles and more runs as several launches, each writing its
+    own partials. K = 1 and small whole numbers: every partial and their sum
+    (below 2^53, in double) are exact, so the result equals the closed form
+    sum_b e_b (sum_m a_bm)(sum_n b_bn), rounded once to the data type. E is
+    one value per batch entry, broadcast over rows and columns (stride 0)."""
+    from trntensor_amd.hip import engine
+
+    g = torch.Generator(device="cuda").manual_seed(batch + M + N)
+    A, B, E = (torch.randint(1, 4, s, generator=g, device="cuda").to(dt) for s in ((batch, M), (batch, N), (batch,)))
+    out = torch.full((), float("nan"), dtype=dt, device="cuda")
+    engine.gemm_dot(False, False, M, N, 1, A, 1, M, B, N, N, batch, M, N, E, [0, 0, 0, 0, 1], None, None, 1.0, 0.0,
+                    None, out)
+    want = (E.double() * A.double().sum(1) * B.double().sum(1)).sum()
+    assert float(out) == float(want.to(dt)), (float(out), float(want))

@@ -47,7 +47,7 @@ __global__ __launch_bounds__(kThreads) void gemm_kernel(GemmArgs g) {
 
     const int64_t tiles = g.tiles_m * g.tiles_n;
     const int64_t total = tiles * g.batch;
-    const int64_t id = xcd_remap(blockIdx.x, total);
+    const int64_t id = DOT ? g.first + xcd_remap(blockIdx.x, gridDim.x) : xcd_remap(blockIdx.x, total);
     const int64_t bat = id / tiles;
     int64_t t = id - bat * tiles;
     // Grouped order: 8 tile-rows sweep each tile-column, so concurrently
@@ -204,7 +204,7 @@ __global__ __launch_bounds__(kThreads) void gemm_kernel(GemmArgs g) {
             }
         }
         const double tot = block256_sum(sum, red);
-        if (threadIdx.x == 0) g.partial[blockIdx.x] = tot;
+        if (threadIdx.x == 0) g.partial[g.first + blockIdx.x] = tot;
         return;
     }
 
@@ -398,7 +398,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     // 60.36 and 60.01 against 60.92 and 61.10 ms on one box (groups of 32:
     // 60.28 and 60.31 ms; of 64: 60.83 and 60.98 ms).
     const int64_t tiles = g.tiles_m * g.tiles_n;
-    const int64_t id = xcd_remap(blockIdx.x, tiles * g.batch);
+    const int64_t id = DOT ? g.first + xcd_remap(blockIdx.x, gridDim.x) : xcd_remap(blockIdx.x, tiles * g.batch);
     const int64_t bat = id / tiles;
     const int64_t rem = id - bat * tiles;
     constexpr int64_t kRowGroup = 16;
@@ -657,7 +657,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
             else dot(std::false_type{}, std::false_type{});
         }
         const double tot = block256_sum(sum, red);
-        if (tid == 0) g.partial[blockIdx.x] = tot;
+        if (tid == 0) g.partial[g.first + blockIdx.x] = tot;
         return;
     } else {
         directb_store<T, FULLM, false, FM>(g, acc, bat, m0, tn);
@@ -982,6 +982,20 @@ int device_cus() {
     return cus[dev];
 }
 
+// Runs launch(workgroups) for `total` tiles. The dot epilogue takes more than a
+// launch may have as several launches, each writing its own range of the
+// partials from g.first up (a dot of 2^24 tiles in one launch left partials
+// unwritten). Products that store D never get here with so many: the tile
+// choice leaves them to kernels that split the product.
+template <bool DOT, typename F>
+static void launch_tiles(GemmArgs& g, int64_t total, F launch) {
+    int64_t n = total;
+    for (g.first = 0; g.first < total; g.first += n) {
+        if (DOT) n = std::min(total - g.first, kMaxGrid);
+        launch(dim3((unsigned)n));
+    }
+}
+
 template <typename T, bool DOT>
 static int launch_directb(GemmArgs& g, bool ta, bool tb, bool nt, hipStream_t st) {
     constexpr int BN = 64 * (16 / sizeof(T));
@@ -1019,7 +1033,8 @@ static int launch_directb(GemmArgs& g, bool ta, bool tb, bool nt, hipStream_t st
         else hipLaunchKernelGGL((gemm_directb_persistent_kernel<T, true, false, false>), grid, block, 0, st, g);
         return check_launch("tt_gemm");
     }
-    const dim3 grid((unsigned)total), block(kThreads);
+    const dim3 block(kThreads);
+    launch_tiles<DOT>(g, total, [&](dim3 grid) {
 #define TT_DIRECTB_CASE(F, A_T, B_T, N_T)                         \
     if (full == F && ta == A_T && tb == B_T && nt == N_T)         \
         hipLaunchKernelGGL((gemm_directb_kernel<T, F, A_T, B_T, N_T, DOT>), grid, block, 0, st, g);
@@ -1032,6 +1047,7 @@ static int launch_directb(GemmArgs& g, bool ta, bool tb, bool nt, hipStream_t st
 #undef TT_DIRECTB_TB
 #undef TT_DIRECTB_NT
 #undef TT_DIRECTB_CASE
+    });
     return check_launch("tt_gemm");
 }
 
@@ -1099,7 +1115,8 @@ static int launch_tile(GemmArgs& g, bool ta, bool tb, hipStream_t st) {
     const int64_t total = g.tiles_m * g.tiles_n * g.batch;
     if (total > 0x7fffffffLL) return set_error(TT_UNSUPPORTED, "tt_gemm: %lld tiles exceed one launch", (long long)total);
     const bool full = g.M % BM == 0 && g.N % BN == 0;
-    dim3 grid((unsigned)total), block(kThreads);
+    const dim3 block(kThreads);
+    launch_tiles<DOT>(g, total, [&](dim3 grid) {
 #define TT_GEMM_CASE(TA, TB, F) \
     if (ta == TA && tb == TB && full == F) hipLaunchKernelGGL((gemm_kernel<T, BM, BN, FM, FN, TA, TB, F, DOT, NBUF, BK>), grid, block, 0, st, g);
     TT_GEMM_CASE(false, false, false)
@@ -1111,6 +1128,7 @@ static int launch_tile(GemmArgs& g, bool ta, bool tb, hipStream_t st) {
     TT_GEMM_CASE(true, true, false)
     TT_GEMM_CASE(true, true, true)
 #undef TT_GEMM_CASE
+    });
     return check_launch("tt_gemm");
 }
 

@@ -17,7 +17,7 @@ struct GemmArgs {
     int64_t tiles_m, tiles_n;
     double alpha, beta;
     // Dot epilogue: instead of storing D, each workgroup writes
-    // sum_{m,n} D[m,n] * E(m,n) to partial[workgroup], with
+    // sum_{m,n} D[m,n] * E(m,n) to partial[first + workgroup], with
     // E(m,n) = E1[off1] * (E2 ? E2[off2] : 1), off = m_hi*s[0] + m_lo*s[1] +
     // n_hi*s[2] + n_lo*s[3] + batch*s[4], (m_hi, m_lo) = divmod(m, mdiv.d),
     // (n_hi, n_lo) = divmod(n, ndiv.d).
@@ -26,6 +26,7 @@ struct GemmArgs {
     int64_t e1s[5], e2s[5];
     FastDiv mdiv, ndiv;
     double* partial;
+    int64_t first;  // first tile of this launch (dot epilogue)
 };
 
 // A product with more tiles than a launch may have workgroups runs as two,
