@@ -67,3 +67,20 @@ def test_mp2_copy_rule(hip, dtype, shape):
         vals.append(float(e))
     assert vals[0] == vals[1]
     assert rel(vals[0], cpu_ref.mp2_energy(B.double(), eo.double(), ev.double())) <= TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("deterministic", [True, False])
+def test_mp2_more_units_than_a_grid(hip, dtype, deterministic):
+    """5793 occupied orbitals are 16782321 pairs, more workgroups than one
+    launch may have: the units run as several launches. One virtual and one
+    auxiliary function, so E = sum_ij (b_i b_j)^2 / (e_i + e_j - 2 e_a); the
+    shards (each within one launch) sum to the same energy."""
+    nocc = 5793
+    B, eo, ev = (x.cuda() for x in inputs(nocc, 1, 1, dtype, 11))
+    got = float(hip._hip_mp2_energy(B, eo, ev, deterministic=deterministic))
+    b2, o = B.double().reshape(-1) ** 2, eo.double()
+    want = float((b2[:, None] * b2[None, :] / (o[:, None] + o[None, :] - 2.0 * ev.double())).sum())
+    assert rel(got, want) <= TOL[dtype]
+    parts = sum(float(hip._hip_mp2_energy_shard(B, eo, ev, r, 3, deterministic=deterministic)) for r in range(3))
+    assert rel(parts, want) <= TOL[dtype]
