@@ -81,6 +81,13 @@ def test_mp2_workspace_holds_a_row_padded_copy_for_unaligned_naux(lib):
         for naux, pitch in ((1199, 1200), (1190, 1200), (1201, 1216), (1, 16)):
             pad = (64 * 320 * pitch * elem + 255) // 256 * 256
             assert lib.tt_mp2_energy_workspace_bytes(code, 64, 320, naux) == part + pad
+    # below nocc * nvir = 7000 no copy is made, and none is asked for
+    for nocc, nvir, naux, copy in ((21, 150, 555, 0), (5, 19, 1 << 20, 0), (70, 99, 33, 0), (70, 100, 33, 1)):
+        nblk = (nvir + 63) // 64
+        units = nocc * (nocc + 1) // 2 * (nblk * (nblk + 1) // 2)
+        room = ((units + 1) * 8 + 255) // 256 * 256
+        pad = (nocc * nvir * ((naux + 15) // 16 * 16) * 8 + 255) // 256 * 256
+        assert lib.tt_mp2_energy_workspace_bytes(1, nocc, nvir, naux) == room + copy * pad
     assert lib.tt_mp2_energy_workspace_bytes(1, 0, 320, 1199) == 256
     # Both entry points accept the partials' size for any naux: below it they refuse.
     dummy = ctypes.c_void_p(256)

@@ -83,11 +83,12 @@ def test_force_backend_env(monkeypatch):
 
 class _FakeMp2Lib:
     """tt_mp2_energy_workspace_bytes with the library's sizes: partials for
-    the work units plus, for naux off a multiple of 16, the padded copy."""
+    the work units plus, for naux off a multiple of 16 from nocc * nvir = 7000
+    on, the padded copy."""
 
     def tt_mp2_energy_workspace_bytes(self, code, nocc, nvir, naux):
         part = 8 * (nocc * (nocc + 1) // 2 * 3 + 1)
-        pad = 0 if naux % 16 == 0 else nocc * nvir * ((naux + 15) // 16 * 16) * 8
+        pad = 0 if naux % 16 == 0 or nocc * nvir < 7000 else nocc * nvir * ((naux + 15) // 16 * 16) * 8
         return part + pad
 
 
@@ -107,15 +108,19 @@ def test_mp2_workspace_falls_back_to_partials_on_oom():
 
         return alloc
 
-    full = lib.tt_mp2_energy_workspace_bytes(1, 4, 100, 1199)
-    part = lib.tt_mp2_energy_workspace_bytes(1, 4, 100, 1200)
+    full = lib.tt_mp2_energy_workspace_bytes(1, 70, 100, 37)
+    part = lib.tt_mp2_energy_workspace_bytes(1, 70, 100, 48)
     assert full > part
-    ws, nb = dispatch._mp2_workspace(lib, 1, 4, 100, 1199, None, _alloc=alloc_oom_above(part))
+    ws, nb = dispatch._mp2_workspace(lib, 1, 70, 100, 37, None, _alloc=alloc_oom_above(part))
     assert nb == part and ws.numel() == part and asked == [full, part]
     asked.clear()
-    ws, nb = dispatch._mp2_workspace(lib, 1, 4, 100, 1199, None, _alloc=alloc_oom_above(full))
+    ws, nb = dispatch._mp2_workspace(lib, 1, 70, 100, 37, None, _alloc=alloc_oom_above(full))
     assert nb == full and ws.numel() == full and asked == [full]
     asked.clear()
-    # naux a multiple of 16: no copy is asked for.
-    ws, nb = dispatch._mp2_workspace(lib, 1, 4, 100, 1200, None, _alloc=alloc_oom_above(full))
+    # naux a multiple of 16, or a molecule below the copy's rule: no copy is asked for.
+    ws, nb = dispatch._mp2_workspace(lib, 1, 70, 100, 48, None, _alloc=alloc_oom_above(full))
+    assert nb == part and asked == [part]
+    asked.clear()
+    part = lib.tt_mp2_energy_workspace_bytes(1, 4, 100, 48)
+    ws, nb = dispatch._mp2_workspace(lib, 1, 4, 100, 37, None, _alloc=alloc_oom_above(full))
     assert nb == part and asked == [part]

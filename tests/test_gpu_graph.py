@@ -119,16 +119,16 @@ def test_einsum_graph_replays(hip, sub, shapes, kw):
         assert torch.equal(res, want), (sub, k, (res.double() - want.double()).abs().max().item())
 
 
-@pytest.mark.parametrize("naux", [96, 37])
-def test_mp2_energy_graph_replays(hip, naux):
-    """The public mp2_energy recorded once under torch.cuda.graph: with naux
-    37 the call stages B into its workspace with rows padded to 48 elements
-    (a copy kernel, then the energy and the fixed-order sum), with naux 96 it
-    runs on B as given. Each replay, with new inputs and eager work in
+@pytest.mark.parametrize("nocc,naux", [(10, 96), (10, 37), (54, 37)])
+def test_mp2_energy_graph_replays(hip, nocc, naux):
+    """The public mp2_energy recorded once under torch.cuda.graph: with 54
+    occupied orbitals (nocc * nvir = 7020) and naux 37 the call stages B into
+    its workspace with rows padded to 48 elements (a copy kernel, then the
+    energy and the fixed-order sum), otherwise it runs on B as given. Each replay, with new inputs and eager work in
     between, equals an eager call bitwise."""
     import trntensor_amd as tt
 
-    B, eo, ev = _inputs(0, naux=naux)
+    B, eo, ev = _inputs(0, nocc=nocc, naux=naux)
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(side):
@@ -139,13 +139,13 @@ def test_mp2_energy_graph_replays(hip, naux):
     with torch.cuda.graph(graph):
         res = tt.mp2_energy(B, eo, ev)
     for k in range(3):
-        src = _inputs(k + 1, naux=naux)
+        src = _inputs(k + 1, nocc=nocc, naux=naux)
         B.copy_(src[0])
         eo.copy_(src[1])
         ev.copy_(src[2])
         torch.cuda.synchronize()
         want = float(tt.mp2_energy(B, eo, ev))
-        print(f"mp2_energy graph naux={naux} replay {k}", flush=True)
+        print(f"mp2_energy graph nocc={nocc} naux={naux} replay {k}", flush=True)
         graph.replay()
         torch.cuda.synchronize()
-        assert float(res) == want, (naux, k, float(res), want)
+        assert float(res) == want, (nocc, naux, k, float(res), want)

@@ -647,9 +647,9 @@ static int64_t mp2_ntasks(int64_t nocc, int64_t nvir) {
 }
 
 // Workspace layout: the per-unit partials (plus one double), then, when naux
-// is not a multiple of the stage depth, room for a copy of B whose rows are
-// padded with zeros to mp2_pitch(naux) elements. The copy is made where each
-// row is read often enough (mp2_copy_pays).
+// is not a multiple of the stage depth and each row is read often enough
+// (mp2_copy_pays), room for a copy of B whose rows are padded with zeros to
+// mp2_pitch(naux) elements.
 //
 // The stages of a row start at multiples of 16 elements from the row start.
 // With naux a multiple of 16 (and B's base so aligned) every stage is a whole
@@ -666,20 +666,20 @@ static size_t mp2_partials_bytes(int64_t nocc, int64_t nvir) {
 
 static int64_t mp2_pitch(int64_t naux) { return (naux + kMp2StageK - 1) / kMp2StageK * kMp2StageK; }
 
-static size_t mp2_pad_bytes(int dtype, int64_t nocc, int64_t nvir, int64_t naux) {
-    if (naux <= 0 || naux % kMp2StageK == 0 || nocc <= 0 || nvir <= 0) return 0;
-    const unsigned __int128 b =
-        (unsigned __int128)nocc * (unsigned __int128)nvir * (unsigned __int128)mp2_pitch(naux) * (dtype == TT_F32 ? 4u : 8u);
-    if (b > (unsigned __int128)(SIZE_MAX / 4)) return SIZE_MAX / 4;
-    return (((size_t)b + 255) / 256) * 256;
-}
-
 // Whether the padded copy pays: a row of B is read about nocc * nvir / 64
 // times, the copy costs one pass over B. us on B as given / with the copy,
 // fp32, fp64: nocc 21, nvir 150, naux 555 (nocc * nvir 3150) 85 / 93, 145 /
 // 155; 30, 200, 600 padded to 608 (6000) 280 / 281, 516 / 521; 44, 175, 653
 // (7700) 417 / 409, 770 / 770; 48, 295, 269 (14160) 606 / 588, 1134 / 1104.
 static bool mp2_copy_pays(int64_t nocc, int64_t nvir) { return nocc * nvir >= 7000; }
+
+static size_t mp2_pad_bytes(int dtype, int64_t nocc, int64_t nvir, int64_t naux) {
+    if (naux <= 0 || naux % kMp2StageK == 0 || nocc <= 0 || nvir <= 0 || !mp2_copy_pays(nocc, nvir)) return 0;
+    const unsigned __int128 b =
+        (unsigned __int128)nocc * (unsigned __int128)nvir * (unsigned __int128)mp2_pitch(naux) * (dtype == TT_F32 ? 4u : 8u);
+    if (b > (unsigned __int128)(SIZE_MAX / 4)) return SIZE_MAX / 4;
+    return (((size_t)b + 255) / 256) * 256;
+}
 
 // src (rows x naux, contiguous) -> dst (rows x pitch), zero in columns naux
 // and beyond. One workgroup per row (grid-stride); each thread forms V
@@ -714,7 +714,7 @@ static int mp2_typed(int64_t nocc, int64_t nvir, int64_t naux, const void* B, co
     // aligned, which the copy's 16-byte stores and the stage alignment need).
     const size_t part = mp2_partials_bytes(nocc, nvir);
     const size_t pad = mp2_pad_bytes(sizeof(T) == 4 ? TT_F32 : TT_F64, nocc, nvir, naux);
-    if (pad > 0 && mp2_copy_pays(nocc, nvir) && ws_bytes >= part && ws_bytes - part >= pad && (reinterpret_cast<uintptr_t>(ws) & 255) == 0) {
+    if (pad > 0 && ws_bytes >= part && ws_bytes - part >= pad && (reinterpret_cast<uintptr_t>(ws) & 255) == 0) {
         T* Bp = reinterpret_cast<T*>(static_cast<char*>(ws) + part);
         const int64_t rows = nocc * nvir, pitch = mp2_pitch(naux);
         hipLaunchKernelGGL(mp2_pad_rows_kernel<T>, dim3((unsigned)(rows < 65536 ? rows : 65536)), dim3(256), 0, st,

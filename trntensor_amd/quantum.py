@@ -30,10 +30,11 @@ def mp2_energy(B: torch.Tensor, eps_occ: torch.Tensor, eps_vir: torch.Tensor) ->
     (trntensor/quantum.py:21-84, 94-99); with one dtype throughout that is
     B's dtype.
 
-    Device memory: when naux is not a multiple of 16 the call also takes a
-    row-padded copy of B (as large as B) for its duration, which makes it
-    5-7% faster; if the device cannot hold the copy, the call runs on B as
-    given with only the per-work-unit partials as workspace.
+    Device memory: when naux is not a multiple of 16 and nocc * nvir reaches
+    7000 the call also takes a row-padded copy of B (as large as B) for its
+    duration, which makes it up to 4% faster; if the device cannot hold the
+    copy, the call runs on B as given with only the per-work-unit partials as
+    workspace.
     """
     if B.dim() != 3:
         raise ValueError(f"B must be 3D (nocc, nvir, naux); got shape {tuple(B.shape)}")
