@@ -263,3 +263,36 @@ def test_gemm_dot_more_tiles_than_a_grid(hip, dt, batch, M, N):
                     None, out)
     want = (E.double() * A.double().sum(1) * B.double().sum(1)).sum()
     assert float(out) == float(want.to(dt)), (float(out), float(want))
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("M,N,K,batch", [(3701, 1179, 3, 1), (193, 161, 16, 150), (42, 50003, 13, 1),
+                                         (90007, 5, 5, 1), (70001, 36, 1, 1), (243, 17, 15, 400),
+                                         (61, 97, 104, 700), (67, 255, 128, 200), (130, 63, 17, 300)])
+def test_gemm_f32_short_k(hip, ta, tb, M, N, K, batch):
+    """Sums of at most 16 terms, for which wide tiles take the well-filled
+    grids, and the tiles up to K = 128: against float64 torch, operands and D in
+    NaN buffers, and bitwise against the last row computed by itself (32 x 32
+    tiles)."""
+    from trntensor_amd.hip import engine
+
+    dt = torch.float32
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    A = torch.randn(batch, M, K, generator=g, dtype=torch.float64, device="cuda").to(dt)
+    B = torch.randn(batch, K, N, generator=g, dtype=torch.float64, device="cuda").to(dt)
+    sa, sb = A.transpose(1, 2) if ta else A, B.transpose(1, 2) if tb else B
+    lda, ldb = sa.shape[2] + 1, sb.shape[2] + 1
+    Ab, sA, _ = embed(sa, lda, 1, dt)
+    Bb, sB, _ = embed(sb, ldb, 1, dt)
+    C = torch.randn(batch, M, N, generator=g, dtype=torch.float64, device="cuda").to(dt)
+    for with_c in (False, True):
+        Db, sD, D = embed(torch.full((batch, M, N), float("nan")), N + 1, 1, dt)
+        engine.gemm(ta, tb, M, N, K, Ab, lda, sA, Bb, ldb, sB, Db, N + 1, sD, batch, 1.5, 0.5 if with_c else 0.0,
+                    C if with_c else None, N, M * N, a_off=1, b_off=1, d_off=1)
+        ref = 1.5 * torch.bmm(A.double(), B.double()) + (0.5 * C.double() if with_c else 0.0)
+        assert float((D.double() - ref).abs().max() / ref.abs().max()) <= TOL[dt]
+        assert int(torch.isnan(Db).sum()) == Db.numel() - batch * M * N
+        P = torch.empty(batch, 1, N, dtype=dt, device="cuda")
+        engine.gemm(ta, tb, 1, N, K, Ab, lda, sA, Bb, ldb, sB, P, N, N, batch, 1.5, 0.5 if with_c else 0.0,
+                    C[:, M - 1] if with_c else None, N, M * N, a_off=1 + (M - 1 if ta else (M - 1) * lda), b_off=1)
+        assert torch.equal(P[:, 0], D[:, M - 1])

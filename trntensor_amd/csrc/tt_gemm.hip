@@ -103,9 +103,12 @@ __global__ __launch_bounds__(kThreads) void gemm_kernel(GemmArgs g) {
         if (edge_m) sa.align(m0, g.M);
         if (edge_n) sb.align(n0, g.N);
     };
-    auto compute = [&](int buf) __attribute__((always_inline)) {
+    // The stage's 16-k passes, of which the last, partial stage of a deep-stage
+    // kernel runs only those that K reaches.
+    auto compute = [&](int buf, int64_t left) __attribute__((always_inline)) {
 #pragma unroll
         for (int kk = 0; kk < BK / 16; ++kk) {
+            if (kk > 0 && 16 * kk >= left) break;
             T fa[FM][4], fb[FN][4];
 #pragma unroll
             for (int i = 0; i < FM; ++i) SA::frag(bufA(buf), wm0 + 16 * i, lane, kk, fa[i]);
@@ -140,7 +143,7 @@ __global__ __launch_bounds__(kThreads) void gemm_kernel(GemmArgs g) {
     int64_t kt = 0;
     for (; kt + 1 < nfull; ++kt) {
         load((kt + 1) * BK);
-        compute(cur(kt));
+        compute(cur(kt), BK);
         __builtin_amdgcn_sched_barrier(0);
         align();
         if (NBUF == 1) __syncthreads();
@@ -150,7 +153,7 @@ __global__ __launch_bounds__(kThreads) void gemm_kernel(GemmArgs g) {
     for (; kt < nk; ++kt) {
         const bool more = kt + 1 < nk;
         if (more) load_tail((kt + 1) * BK);
-        compute(cur(kt));
+        compute(cur(kt), g.K - kt * BK);
         __builtin_amdgcn_sched_barrier(0);
         if (NBUF == 1) __syncthreads();
         if (more) store(next(kt));
@@ -1163,21 +1166,45 @@ static int gemm_f32(GemmArgs& g, bool ta, bool tb, hipStream_t st) {
     // 786432 x 512 TN 452/787/470/535/623; 80 x 200000 x 300 TN
     // -/156/150/170/160.
     const double never = 1e300;
+    auto tiles = [&](int64_t bm, int64_t bn) { return ((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn) * g.batch; };
     auto cost = [&](int64_t bm, int64_t bn, double per_output, double one, double two) {
-        const int64_t n = ((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn) * g.batch;
+        const int64_t n = tiles(bm, bn);
         if (n > kMaxGrid && bm > 32) return never;  // not one launch; the 32 x 32 tiles take several
         const int64_t rounds = (n + cus - 1) / cus;
         return (double)(rounds * bm * bn) * per_output * (rounds == 1 ? one : rounds == 2 ? two : 1.0);
     };
     const bool rows_ok = !ta || g.M >= 4, cols_ok = tb || g.N >= 4;  // a 16-byte piece along a row-contiguous operand
+    // Short sums do not pay for deep stages and their prologue. K of at most
+    // one 16-deep stage: every tile costs about the same per workgroup, whatever
+    // its area (32 x 32 2.1 ns, 64 x 128 with 16-deep stages 6 ns, chip-wide), so
+    // the wide ones win where they are few and well filled. us, 64 x 128 / best of
+    // the others (the 64-deep tiles had lost these to the kernels before them):
+    // 3706 x 1179 x 3 9.0 / 14.3, 198 x 161 x 5 x 1356 61 / 76, 43 x 183720 x 3
+    // 14.3 / 17.4, 72 x 234521 x 1 25 / 37; 256 x 64 / 32 x 32 without C: 169059 x
+    // 5 x 5 8.9 / 12.2, 113627 x 36 x 3 9.6 / 12.0, 242 x 17 x 4 x 365 7.9 / 8.6.
+    if (g.K <= 16) {
+        const int64_t n32 = tiles(32, 32), wide = tiles(64, 128), tall = tiles(256, 64);
+        if (g.N <= 64 && !g.C && n32 >= 2560 && n32 >= 7 * tall * ((g.N + 31) / 32) && tall <= kMaxGrid)
+            return launch_tile<float, 256, 64, 4, 4, false>(g, ta, tb, st);
+        // Half-empty tiles (M <= 32) that read C wait for more rounds: 20 x 71286 x
+        // 8 with C 8.5 / 7.4 us, 16 x 163083 x 11 11.4 / 13.3.
+        if (n32 >= (g.C && g.M <= 32 ? 4096 : 1280) && n32 >= 3 * wide && wide <= kMaxGrid)
+            return launch_tile<float, 64, 128, 2, 4, false>(g, ta, tb, st);
+    }
+    // Up to K = 128 the 64 x 128 tile with 16-deep stages stays a candidate, and
+    // the 32 x 32 tile's single 128-deep stage (K > 64) leaves fewer workgroups on
+    // a CU: 60 x 96 x 104 x 704 NT with C 22 / 28 us.
+    const double wide16 = g.K > 16 && g.K <= 128 ? cost(64, 128, 1.02, 1.3, 1.1) : never;
     const double direct = rows_ok && !tb && g.N % 256 == 0 ? cost(64, 256, 0.97, 1.1, 1.0) : never;
     const double tall = rows_ok && cols_ok && g.K > 0 ? cost(128, 128, 1.0, 1.05, 1.0) : never;
     const double mid = rows_ok && cols_ok && g.K > 0 ? cost(64, 128, 1.04, 1.05, 1.0) : never;
     const double square = cost(64, 64, 1.1, 1.25, 1.1);
-    const double small = cost(32, 32, ta && !tb ? 1.5 : tb && !ta ? 1.25 : 1.35, 1.1, 1.1);
-    const double best = std::min({direct, tall, mid, square, small});
+    const bool deep = g.K > 64 && g.K <= 128 && tiles(32, 32) > 2 * cus;
+    const double small = cost(32, 32, (ta && !tb ? 1.5 : tb && !ta ? 1.25 : 1.35) * (deep ? 1.2 : 1.0), 1.1, 1.1);
+    const double best = std::min({direct, tall, mid, square, small, wide16});
     if (best == small) return gemm_small_launch(TT_F32, ta, tb, g, st);
     if (best == square) return launch_tile<float, 64, 64, 2, 2, false, 1, 64>(g, ta, tb, st);
+    if (best == wide16) return launch_tile<float, 64, 128, 2, 4, false>(g, ta, tb, st);
     if (best == direct) return launch_directb<float, false>(g, ta, false, g.M <= 64 && (g.batch == 1 || g.sB != 0), st);
     return gemm_mid_f32_launch(ta, tb, best == tall, g, st);
 }
