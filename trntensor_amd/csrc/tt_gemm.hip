@@ -1091,7 +1091,10 @@ static int gemm_f64(GemmArgs& g, bool ta, bool tb, hipStream_t st) {
     const bool nt = g.M <= 64 && (g.batch == 1 || g.sB != 0);  // B is read once
     const int64_t cus = device_cus();
     auto up = [](int64_t n, int64_t t) { return (n + t - 1) / t; };
-    const double cols = (double)(up(g.N, 32) * 32) / (double)(up(g.N, 128) * 128);
+    // A wave past the last column does not give all of its share back where K is
+    // long: 292 x 9 x 190 x 199 (one live wave of four) 22 us on 64 rows, 31 on 32.
+    double cols = (double)(up(g.N, 32) * 32) / (double)(up(g.N, 128) * 128);
+    if (g.K > 32) cols = std::max(cols, 0.6);
     auto direct = [&](int64_t fm, double per_output) {
         const int64_t n = up(g.M, 16 * fm) * up(g.N, 128) * g.batch;
         if (n > kMaxGrid) return 1e300;  // not one launch; the 32 x 32 tiles take several
@@ -1100,12 +1103,18 @@ static int gemm_f64(GemmArgs& g, bool ta, bool tb, hipStream_t st) {
         return (double)(rounds * 16 * fm * 128) * share * per_output * (rounds == 1 ? 1.6 : 1.0);
     };
     const int64_t sr = up(up(g.M, 32) * up(g.N, 32) * g.batch, cus);
-    const double small = (double)(sr * 32 * 32) * 1.4 * (sr <= 2 ? 1.1 : 1.0);
+    // A short sum leaves most of a 64-deep stage empty: 318 x 3602 x 7 NT 7.7 us
+    // on 32 x 32, 5.8 on 32 x 128; 8 x 68679 x 1 8.9 / 5.6.
+    const bool empty = g.K <= 32 && g.N > 32 && sr > 4;
+    const double small = (double)(sr * 32 * 32) * 1.4 * (sr <= 2 ? 1.1 : 1.0) * (empty ? 1.4 : 1.0);
     const double d4 = direct(4, 1.0), d3 = direct(3, 1.04), d2 = direct(2, 1.1);
     // A whole 16-byte piece along a row-contiguous operand, else 32 x 32 tiles
     // (100000 x 1 x 300 51 against 118 us on 256 x 64 LDS tiles).
     const bool direct_ok = g.N >= 2 && (!ta || g.M >= 2);
-    if (!direct_ok || (small < d4 && small < d3 && small < d2)) return gemm_small_launch(TT_F64, ta, tb, g, st);
+    // One 32 x 32 tile per batch entry, where the direct-B tiles have one live
+    // wave: 12 x 32 x 32 x 1432 NT 6.6 us against 8.0 on 32 x 128.
+    const bool one = g.M <= 32 && g.N <= 32 && g.K > 16;
+    if (!direct_ok || one || (small < d4 && small < d3 && small < d2)) return gemm_small_launch(TT_F64, ta, tb, g, st);
     if (d2 < d4 && d2 < d3) return launch_directb_rows(g, ta, tb, nt, 2, st);
     if (d3 < d4) return launch_directb_rows(g, ta, tb, nt, 3, st);
     return launch_directb<double, false>(g, ta, tb, nt, st);
