@@ -88,6 +88,39 @@ def test_gemm_dot_unaligned_ragged(hip, dt, ta, tb, M, N, K):
     assert abs(float(out) - float((X * E).sum())) <= TOL[dt] * scale
 
 
+@pytest.mark.parametrize("ta,tb", [(False, True), (True, False)])
+@pytest.mark.parametrize("M,N", [(12 * 17, 9), (9, 12 * 17), (12 * 11, 10 * 13), (300, 6 * 7), (1, 130), (70, 1)])
+@pytest.mark.parametrize("K", [5, 200])
+def test_gemm_dot_orientation(hip, ta, tb, M, N, K):
+    """fp64 dots run as given or exchanged, after their tiles and E's strides:
+    E contiguous along n, along m, and as an outer product of two factors
+    whose letters interleave (m = (a, b), n = (i, j), E = X[a, i] Y[b, j]),
+    each against float64 torch."""
+    from trntensor_amd.hip import engine
+
+    dt = torch.float64
+    g = torch.Generator().manual_seed(M + 7 * N + K)
+    A = torch.randn(1, M, K, generator=g, dtype=dt)
+    B = torch.randn(1, K, N, generator=g, dtype=dt)
+    E = torch.randn(M, N, generator=g, dtype=dt)
+    sa, sb = A.transpose(1, 2) if ta else A, B.transpose(1, 2) if tb else B
+    Ad, Bd = sa.contiguous().cuda(), sb.contiguous().cuda()
+    ml = next(d for d in (17, 11, 9, 1) if M % d == 0)
+    nl = next(d for d in (13, 7, 1) if N % d == 0)
+    X = torch.randn(M // ml, N // nl, generator=g, dtype=dt)
+    Y = torch.randn(ml, nl, generator=g, dtype=dt)
+    outer = (X[:, None, :, None] * Y[None, :, None, :]).reshape(M, N)
+    forms = [(E, E, [0, N, 0, 1, 0], None, None, M, N), (E, E.t().contiguous(), [0, 1, 0, M, 0], None, None, M, N),
+             (outer, X, [N // nl, 0, 1, 0, 0], Y, [0, nl, 0, 1, 0], ml, nl),
+             (outer, X.t().contiguous(), [1, 0, M // ml, 0, 0], Y.t().contiguous(), [0, 1, 0, ml, 0], ml, nl)]
+    P = torch.bmm(A, B)[0]
+    for k, (full, e1, s1, e2, s2, m_lo, n_lo) in enumerate(forms):
+        out = torch.full((), float("nan"), dtype=dt, device="cuda")
+        engine.gemm_dot(ta, tb, M, N, K, Ad, sa.shape[2], 0, Bd, sb.shape[2], 0, 1, m_lo, n_lo, e1.cuda(), s1,
+                        None if e2 is None else e2.cuda(), s2, 1.0, 0.0, None, out)
+        assert abs(float(out) - float((P * full).sum())) <= TOL[dt] * float((P * full).abs().sum()), k
+
+
 @pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
 @pytest.mark.parametrize("M,N,K", [(33, 47, 21), (500, 700, 37), (1030, 1025, 18), (2050, 2049, 17), (1, 1, 16), (17, 3, 100)])
 def test_gemm_dd_tiles(hip, ta, tb, M, N, K):

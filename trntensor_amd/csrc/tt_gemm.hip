@@ -1402,11 +1402,26 @@ extern "C" int tt_gemm_dot(int dtype, int transA, int transB, int64_t M, int64_t
         g.ndiv = make_fastdiv((uint32_t)nlo);
         g.partial = static_cast<double*>(workspace);
         bool ta = transA != 0, tb = transB != 0;
-        // fp64 runs on 64 x 128 tiles: where fewer of them cover the product
-        // the other way round, X^T = op(B)^T op(A)^T is formed instead, E read
-        // with its row and column parts exchanged (16900 x 900: 1995 tiles
-        // instead of 2120).
-        if (dtype == TT_F64 && ((N + 63) / 64) * ((M + 127) / 128) < ((M + 63) / 64) * ((N + 127) / 128)) {
+        // fp64 runs on 64 x 128 tiles. X^T = op(B)^T op(A)^T is formed instead,
+        // E read with its row and column parts exchanged, where that costs less:
+        // the busiest CU's tiles times their K, plus 60 k for what a tile costs
+        // besides, plus 50 k where the lanes, which run along the columns, read E
+        // or E2 with a stride of more than 16 elements (a cache line); with equal
+        // costs the fewer tiles. us, as given / exchanged: E and E2 an outer product
+        // with strided lanes as given, not when exchanged: 16900 x 900 x 450 (2120 /
+        // 1995 tiles) 273 / 238, 16384 x 1024 x 512 (2048 / 2048) 265 / 256, 40000 x
+        // 256 x 100 (1250 / 1252) 65 / 54, 160000 x 16384 x 800 60.1 / 59.2 ms. E
+        // contiguous along n: 4065 x 21285 x 4 (10688 / 10656) 262 / 469, 1605 x 19235
+        // x 12 124 / 175, 128 x 20254 x 533 80 / 85, 27541 x 256 x 270 84 / 99; but
+        // 19486 x 773 x 417 (9 tiles on a CU / 8) 255 / 224, 16501 x 9 x 70 18 / 13.
+        auto dot_cost = [&](int64_t m, int64_t n, int lane) {
+            auto strided = [&](const int64_t* s) { return s[lane] > 16 || s[lane] < -16; };
+            const int64_t pen = strided(g.e1s) || (E2 && strided(g.e2s)) ? 50 : 0;
+            const int64_t tiles = ((m + 63) / 64) * ((n + 127) / 128) * batch, cus = device_cus();
+            if (tiles > 0x7fffffffLL) return 1e300;  // not launched
+            return (double)((tiles + cus - 1) / cus) * (double)(K + 60 + pen) + 1e-10 * (double)tiles;
+        };
+        if (dtype == TT_F64 && dot_cost(N, M, m_lo > 1 ? 1 : 0) < dot_cost(M, N, n_lo > 1 ? 3 : 2)) {
             std::swap(g.A, g.B);
             std::swap(g.M, g.N);
             std::swap(g.lda, g.ldb);
