@@ -1435,6 +1435,11 @@ extern "C" int tt_gemm_dot(int dtype, int transA, int transB, int64_t M, int64_t
             tb = !ta;
             ta = t;
         }
+        // A contiguous vector is k-contiguous in either form, and as such read in
+        // 16-byte pieces instead of element by element: 1 x 29 x 1332 x 24 TN fp64
+        // 152 -> 94 us, 47 x 1 x 1224 TN fp32 97 -> 60.
+        if (g.N == 1 && !tb && g.ldb == 1) tb = true, g.ldb = std::max<int64_t>(K, 1);
+        if (g.M == 1 && ta && g.lda == 1) ta = false, g.lda = std::max<int64_t>(K, 1);
         const int rc = gemm_dot_dispatch(dtype, ta, tb, g, st, &nparts);
         if (rc != TT_OK) return rc;
     }
