@@ -290,14 +290,16 @@ __global__ __launch_bounds__(256) void strided_transpose_kernel(StridedArgs g, T
     constexpr int RP = 256 / TS;       // tile rows per pass of the 256 threads
     constexpr int NE = TS * TS / 256;  // elements per thread
     __shared__ T tile[TS][TS + 1];
-    const int64_t per = t.tiles_u * t.tiles_v;
-    const int64_t id = t.shared ? xcd_remap(blockIdx.x, gridDim.x) : blockIdx.x;
-    const int64_t z = id / per;
-    const int64_t rem = id - z * per;
-    const int64_t u0 = (rem % t.tiles_u) * TS;
-    const int64_t v0 = (rem / t.tiles_u) * TS;
+    // Tile indices in 32 bits (the launch has fewer than 2^24 tiles).
+    const uint32_t tiles_u = (uint32_t)t.tiles_u, per = tiles_u * (uint32_t)t.tiles_v;
+    const uint32_t id = t.shared ? (uint32_t)xcd_remap(blockIdx.x, gridDim.x) : blockIdx.x;
+    const uint32_t z = id / per;
+    const uint32_t rem = id - z * per;
+    const uint32_t tv = rem / tiles_u;
+    const int64_t u0 = (int64_t)(rem - tv * tiles_u) * TS;
+    const int64_t v0 = (int64_t)tv * TS;
     int64_t za, zd;
-    decode((uint32_t)z, t.bat, za, zd);
+    decode(z, t.bat, za, zd);
     const T* A = static_cast<const T*>(g.A);
     const int lo = threadIdx.x % TS;
     const int hi = threadIdx.x / TS;
