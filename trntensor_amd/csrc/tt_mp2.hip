@@ -26,7 +26,7 @@
 #include <mutex>
 #include <type_traits>
 
-#include "tt_common.hpp"
+#include "tt_gemm.hpp"
 
 namespace tt {
 
@@ -707,6 +707,19 @@ __global__ __launch_bounds__(256) void mp2_pad_rows_kernel(const T* __restrict__
     }
 }
 
+// Whether the narrow forms shorten the launch. With a unit or less per CU they
+// don't where a pair has a full off-diagonal unit (three and more blocks): the
+// launch ends with those, and the kernel with the narrow forms has the slower
+// schedule for them. The same holds in fp64 up to two units per CU from five
+// blocks on, where few units are narrow. us, with / without the narrow forms: 3,
+// 277, 560 fp64 47.2 / 46.7; 5, 130, 400 36.1 / 35.5; 7, 277, 560 73.9 / 71.7; 4, 400,
+// 880 114.6 / 106.9; 6, 345, 880 109.4 / 107.3; but 9, 130, 400 39 / 48; 10, 277, 560
+// 115 / 119; 7, 400, 880 179 / 193; two blocks 8, 90, 320 21 / 30.
+static bool mp2_narrow_pays(size_t elem, int nblk, int64_t units) {
+    const int64_t cus = device_cus();
+    return nblk < 3 || units > (elem == 8 && nblk >= 5 ? 2 * cus : cus);
+}
+
 template <typename T>
 static int mp2_typed(int64_t nocc, int64_t nvir, int64_t naux, const void* B, const void* eo, const void* ev,
                      void* out, void* ws, size_t ws_bytes, int det, hipStream_t st, int64_t first, int64_t count) {
@@ -743,7 +756,7 @@ static int mp2_typed(int64_t nocc, int64_t nvir, int64_t naux, const void* B, co
         hipLaunchKernelGGL(zero_double_kernel, dim3(1), dim3(64), 0, st, w);
     }
     constexpr int BK = kMp2StageK;
-    const bool tail = nvir % kMp2Tile >= 1 && nvir % kMp2Tile <= 32;
+    const bool tail = nvir % kMp2Tile >= 1 && nvir % kMp2Tile <= 32 && mp2_narrow_pays(sizeof(T), g.nblk, count);
     for (int64_t done = 0; done < count; done += g.ntasks) {
         Mp2Args l = g;
         l.first = first + done;
