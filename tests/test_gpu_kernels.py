@@ -90,13 +90,23 @@ def test_gemm_batched_alpha_beta_ld(hip, dt, pad):
 @pytest.mark.parametrize(
     "ta,tb,M,N,K,batch",
     [
-        (False, False, 64, 300, 70, 2),  # 64 x 128 tiles (M <= 64)
-        (True, False, 200, 150, 40, 3),  # 64 x 128 (fp64 batched, K <= 1024; small grid)
-        (False, True, 300, 50, 90, 1),  # 256 x 64 tiles (N <= 64)
-        (True, True, 257, 300, 129, 1),  # 64 x 128 tiles (small grid), ragged edges
-        (False, True, 2700, 2700, 40, 1),  # 128 x 128 tiles (484 of them), ragged edges
-        (False, False, 200, 512, 48, 2),  # direct-B, 16-byte C pieces of two row blocks at a time, ragged M
-        (True, False, 512, 768, 64, 3),  # direct-B, the batched shape family of config 2
+        # 32 x 32 tiles
+        (False, False, 64, 300, 70, 2),
+        (True, False, 200, 150, 40, 3),
+        (False, True, 300, 50, 90, 1),
+        (True, True, 257, 300, 129, 1),
+        (False, False, 200, 512, 48, 2),
+        (True, False, 512, 768, 64, 3),
+        # fp64 direct-B on 48, 32 and 64 rows; fp32 128 x 128, 64 x 64, 64 x 128, 64 x 256 direct-B
+        (False, True, 2700, 2700, 40, 1),
+        (False, False, 17, 60001, 37, 1),
+        (True, False, 64, 60000, 37, 1),
+        (False, False, 4096, 3840, 48, 1),
+        (True, False, 2061, 2051, 70, 1),
+        (False, False, 1999, 3001, 200, 1),
+        (True, True, 1999, 3001, 200, 1),
+        (True, False, 4001, 4003, 200, 1),
+        (False, False, 60, 97, 104, 700),  # fp32: 64 x 128 with 16-deep stages
         (False, False, 4096, 4096, 1024, 1),  # fp32: the 256 x 256 LDS tile (with C: K >= 1024)
         (False, False, 512, 512, 1024, 64),  # fp32: the 256 x 256 LDS tile, batched, with C
     ],
@@ -106,6 +116,17 @@ def test_gemm_d_aliases_c(hip, dt, ta, tb, M, N, K, batch):
     Each row block's C values are loaded before its stores, so every element is
     read before it is overwritten."""
     assert _gemm_case(hip, dt, ta, tb, M, N, K, batch, 1.5, 0.5, True, seed=M + N, alias=True) <= TOL[dt]
+
+
+def _corner(engine, ta, tb, M, N, K, A, lda, sA, B, ldb, sB, bi, alpha, beta, C, ldc):
+    """The last 40 x 40 outputs of batch entry bi as a product of their own,
+    which takes the 32 x 32 tiles whatever kernel the whole product takes."""
+    m, n = min(40, M), min(40, N)
+    r, c = M - m, N - n
+    P = torch.full((m, n), float("nan"), dtype=A.dtype, device=A.device)
+    engine.gemm(ta, tb, m, n, K, A, lda, 0, B, ldb, 0, P, n, 0, 1, alpha, beta, None if C is None else C[bi, r:, c:],
+                ldc, 0, a_off=bi * sA + (r if ta else r * lda), b_off=bi * sB + (c * ldb if tb else c))
+    return P, r, c
 
 
 @pytest.mark.parametrize("dt", [torch.float64, torch.float32])
@@ -119,10 +140,10 @@ def test_gemm_d_aliases_c(hip, dt, ta, tb, M, N, K, batch):
         (True, 50, 1024, 500, 1, 1.0, 0.0, False, 0),  # M < 64, K tail
         (True, 33, 1152, 7, 2, 0.5, 2.0, True, 1),  # one partial stage only
         (True, 1, 256, 31, 1, 1.0, 0.0, False, 0),
-        (True, 64, 1030, 48, 1, 1.0, 0.5, True, 0),  # fp64: partial last column tile; fp32: LDS-staged in both runs
-        (False, 200, 300, 100, 2, 1.5, 0.5, True, 1),  # fp64: partial last column tile, ragged M
-        (False, 130, 2, 33, 1, 1.0, 0.0, False, 0),  # fp64: one tile of two columns
-        # batched, B cached (64-row slabs of A, either layout)
+        (True, 64, 1030, 48, 1, 1.0, 0.5, True, 0),  # partial last column tile
+        (False, 200, 300, 100, 2, 1.5, 0.5, True, 1),  # partial last column tile, ragged M
+        (False, 130, 2, 33, 1, 1.0, 0.0, False, 0),  # one tile of two columns
+        # batched, B cached
         (False, 512, 512, 512, 4, 1.5, 0.5, True, 0),  # the 64 x 512^3 batch's shape
         (True, 512, 512, 512, 3, 1.0, 0.0, False, 0),
         (True, 320, 1536, 512, 2, 1.0, 0.0, False, 0),  # the AO->MO transform's second GEMM
@@ -131,6 +152,12 @@ def test_gemm_d_aliases_c(hip, dt, ta, tb, M, N, K, batch):
         # more than 64 row tiles: rows in groups of 16 slabs sweeping every column tile
         (False, 4160, 512, 48, 1, 1.5, 0.5, True, 0),
         (True, 4200, 768, 40, 2, 1.0, 0.0, False, 1),  # ragged last group and rows
+        # grids that fill the chip: 64-row direct-B tiles (fp64; fp32 64 x 256 where M has many rows)
+        (False, 4096, 3840, 33, 1, 1.5, 0.5, True, 1),  # whole rows, K tail, odd ldc/ldd
+        (True, 4096, 3840, 48, 1, 1.0, 0.0, False, 0),
+        (False, 4090, 3840, 33, 1, 1.5, 0.5, True, 0),  # ragged rows
+        (True, 64, 60160, 37, 1, 1.0, 0.0, False, 0),  # fp64: B read once (non-temporal loads)
+        (True, 50, 60160, 37, 1, 1.5, 0.5, True, 1),
         # fp32, whole 256 x 256 tiles, one per CU: the LDS-staged 256 x 256 tile kernel
         (False, 4096, 4096, 1024, 1, 1.5, 0.5, True, 0),
         (False, 2048, 8192, 32, 1, 1.0, 0.0, False, 0),  # one 32-k stage
@@ -138,13 +165,13 @@ def test_gemm_d_aliases_c(hip, dt, ta, tb, M, N, K, batch):
         (False, 1024, 1024, 1024, 16, 1.5, 0.5, True, 0),  # batched with C, K >= 1024
     ],
 )
-def test_gemm_direct_b_matches_lds_tile(hip, dt, ta, M, N, K, batch, alpha, beta, with_c, ldd_pad):
-    """B row-major, N even (fp64) or a multiple of 256 (fp32): the kernel that
-    loads B straight into the MFMA registers, or, for fp32 problems of whole
-    256 x 256 tiles filling the chip, the 256 x 256 tile. Checked against
-    float64 torch, and bitwise against the LDS-staged tiles, which the same
-    problem takes when B's leading dimension breaks 16-byte alignment (no
-    vector path)."""
+def test_gemm_direct_b_matches_small_tile(hip, dt, ta, M, N, K, batch, alpha, beta, with_c, ldd_pad):
+    """B row-major. Grids that fill the chip: the kernel that loads B straight
+    into the MFMA registers (fp64, and fp32 with N a multiple of 256), or, for
+    fp32 problems of whole, aligned 256 x 256 tiles, the 256 x 256 tile;
+    smaller grids: the 32 x 32 or 64 x 64 tiles. Checked against float64 torch;
+    bitwise with an odd leading dimension of B (fp32: off the 256 x 256 tile);
+    and bitwise against the last 40 x 40 outputs on 32 x 32 tiles."""
     from trntensor_amd.hip import engine
 
     g = torch.Generator().manual_seed(M + N + K + batch + int(ta))
@@ -164,8 +191,8 @@ def test_gemm_direct_b_matches_lds_tile(hip, dt, ta, M, N, K, batch, alpha, beta
     if with_c:
         ref = ref + beta * C[:, :, :N]
     Ad, Cd = A.to(dev, dt), C.to(dev, dt)
-    Bn = B[:, :, :ldb_even].contiguous().to(dev, dt)  # aligned ldb: the direct-B kernel
-    Bo = B[:, :, :ldb_odd].contiguous().to(dev, dt)  # odd ldb: the LDS-staged tiles only
+    Bn = B[:, :, :ldb_even].contiguous().to(dev, dt)
+    Bo = B[:, :, :ldb_odd].contiguous().to(dev, dt)
     outs = []
     for Bd, ldb in ((Bn, ldb_even), (Bo, ldb_odd)):
         D = torch.full((batch, M, ld), float("nan"), dtype=dt, device=dev)
@@ -173,10 +200,14 @@ def test_gemm_direct_b_matches_lds_tile(hip, dt, ta, M, N, K, batch, alpha, beta
                     Cd if with_c else None, ld, M * ld)
         outs.append(D)
     torch.cuda.synchronize()
-    direct, staged = outs[0][:, :, :N], outs[1][:, :, :N]
+    direct, unaligned = outs[0][:, :, :N], outs[1][:, :, :N]
     assert normwise(direct.cpu().double(), ref) <= TOL[dt]
-    assert torch.equal(direct, staged)
+    assert torch.equal(direct, unaligned)
     assert torch.isnan(outs[0][:, :, N:]).all()  # nothing stored past column N
+    for bi in {0, batch - 1}:
+        P, r, c = _corner(engine, ta, False, M, N, K, Ad, lda, a_rows * lda, Bn, ldb_even, K * ldb_even, bi, alpha,
+                          beta, Cd if with_c else None, ld)
+        assert torch.equal(direct[bi, r:, c:], P)
 
 
 @pytest.mark.parametrize(
@@ -190,12 +221,23 @@ def test_gemm_direct_b_matches_lds_tile(hip, dt, ta, M, N, K, batch, alpha, beta
         (True, 128, 256, 16, 1, 1.0, 0.25, True, 0),  # one full stage only
         (False, 192, 200, 64, 1, 1.0, 0.0, False, 0),  # partial last column tile
         (True, 70, 1030, 100, 2, 1.5, 0.5, True, 1),  # partial last column tile, ragged M
+        # grids that fill the chip: the direct-B kernel on 64 rows, whole ...
+        (False, 4096, 3968, 37, 1, 1.0, 0.0, False, 0),
+        (True, 4096, 3968, 64, 1, 1.5, 0.5, True, 1),
+        (True, 64, 60000, 37, 1, 1.0, 0.0, False, 0),  # non-temporal B loads, partial last column tile
+        (False, 64, 60000, 32, 1, 1.5, 0.5, True, 0),
+        # ... or ragged, and on 48 and 32 rows
+        (False, 4000, 3971, 37, 1, 1.5, 0.5, True, 0),
+        (True, 50, 60001, 37, 1, 1.5, 0.5, True, 1),
+        (False, 40, 60001, 37, 1, 1.0, 0.0, False, 0),
+        (True, 20, 60001, 37, 1, 1.5, 0.5, True, 0),
     ],
 )
-def test_gemm_direct_b_k_contiguous_matches_lds_tile(hip, ta, M, N, K, batch, alpha, beta, with_c, ldd_pad):
-    """fp64 with B stored [n][k] (k-contiguous), N even: the
-    direct-B kernel with 16-byte k pieces. Checked against float64 torch, and
-    bitwise against the LDS-staged tiles (reached with an odd ldb)."""
+def test_gemm_direct_b_k_contiguous_matches_small_tile(hip, ta, M, N, K, batch, alpha, beta, with_c, ldd_pad):
+    """fp64 with B stored [n][k] (k-contiguous): the direct-B kernel with
+    16-byte k pieces where the grid fills the chip, else 32 x 32 tiles. Checked
+    against float64 torch, bitwise with an odd ldb, and bitwise against the
+    last 40 x 40 outputs on 32 x 32 tiles."""
     from trntensor_amd.hip import engine
 
     dt = torch.float64
@@ -223,9 +265,13 @@ def test_gemm_direct_b_k_contiguous_matches_lds_tile(hip, ta, M, N, K, batch, al
                     Cd if with_c else None, ld, M * ld)
         outs.append(D)
     torch.cuda.synchronize()
-    direct, staged = outs[0][:, :, :N], outs[1][:, :, :N]
+    direct, unaligned = outs[0][:, :, :N], outs[1][:, :, :N]
     assert normwise(direct.cpu(), ref) <= TOL[dt]
-    assert torch.equal(direct, staged)
+    assert torch.equal(direct, unaligned)
+    for bi in {0, batch - 1}:
+        P, r, c = _corner(engine, ta, True, M, N, K, Ad, lda, a_rows * lda, Bd, ldb, N * ldb, bi, alpha, beta,
+                          Cd if with_c else None, ld)
+        assert torch.equal(direct[bi, r:, c:], P)
     if ld > N:
         assert torch.isnan(outs[0][:, :, N:]).all()  # nothing stored past column N
 
@@ -238,17 +284,16 @@ def test_gemm_direct_b_k_contiguous_matches_lds_tile(hip, ta, M, N, K, batch, al
         (True, False, 128, 384, 37, 3, True),  # K tail, B row-major
         (True, True, 192, 128, 16, 1, False),
         (False, True, 4224, 256, 64, 1, True),  # 66 row tiles: the grouped row order of config 5's GEMM
-        (False, True, 400, 256, 800, 1, True),  # ragged M: config 5's optimal-order dot GEMM, transposed
+        (False, True, 400, 256, 800, 1, True),  # ragged M
         (True, False, 200, 384, 37, 2, False),  # ragged M and K tail, B row-major
         (False, False, 33, 128, 16, 1, True),  # one partial row tile
     ],
 )
-def test_gemm_dot_direct_b_matches_lds_tile(hip, ta, tb, M, N, K, batch, with_e2):
-    """fp64 dot GEMM (sum of op(A) op(B) .* E1 .* E2) with N a multiple of 128
-    (any M; rows past M are left out of the sum): the direct-B kernel's dot
-    epilogue. Against float64 torch, and
-    against the LDS-staged tiles (odd ldb) to 1e-13 relative: the per-tile sums
-    are added in another order."""
+def test_gemm_dot_direct_b_unaligned(hip, ta, tb, M, N, K, batch, with_e2):
+    """fp64 dot GEMM (sum of op(A) op(B) .* E1 .* E2; rows and columns past the
+    matrix are left out of the sum): the direct-B kernel's dot epilogue.
+    Against float64 torch to 1e-13 of the sum of magnitudes, and the same,
+    bitwise, from rows of B that are not 16-byte aligned (odd ldb)."""
     from trntensor_amd.hip import engine
 
     dt = torch.float64
@@ -276,10 +321,10 @@ def test_gemm_dot_direct_b_matches_lds_tile(hip, ta, tb, M, N, K, batch, with_e2
         engine.gemm_dot(ta, tb, M, N, K, A.to(dev), lda, a_rows * lda, Bd, ldb, b_rows * ldb, batch, M, N, E1.to(dev), es,
                         E2.to(dev) if with_e2 else None, es if with_e2 else None, 1.0, 0.0, None, out)
         outs.append(float(out.cpu()))
-    direct, staged = outs
+    direct, unaligned = outs
     scale = float((X.abs() * E1.abs() * (E2.abs() if with_e2 else 1.0)).sum())
     assert abs(direct - ref) <= 1e-13 * scale
-    assert abs(direct - staged) <= 1e-13 * scale
+    assert direct == unaligned
 
 
 def test_gemm_k_zero_is_beta_c(hip):
@@ -432,9 +477,9 @@ def test_gemm_persistent_matches_per_tile_kernel(hip, dt, M, ntiles, K, batch, a
     next tile's first stage loaded during the current tile's last MFMAs), or
     for fp64 with at most two row tiles and N a multiple of 256 its streaming
     variant (64 x 256 tiles, two workgroups per CU).
-    Bitwise equal to the per-tile direct-B kernel, which the same columns take
-    in a launch of fewer tiles (the two keep one MFMA order per output), and
-    checked against float64 torch on sampled columns."""
+    Bitwise equal to the smaller tiles that the same columns take in launches
+    of 16 column tiles (one MFMA order per output), and checked against
+    float64 torch on sampled columns."""
     from trntensor_amd.hip import engine
 
     dev = torch.device("cuda")
@@ -447,7 +492,7 @@ def test_gemm_persistent_matches_per_tile_kernel(hip, dt, M, ntiles, K, batch, a
     B = torch.randn(batch, K, N, generator=g, device=dev, dtype=torch.float64).to(dt)
     D = torch.full((batch, M, N), float("nan"), dtype=dt, device=dev)
     engine.gemm(True, False, M, N, K, A, M, K * M, B, N, K * N, D, N, M * N, batch, alpha)
-    # The same columns in launches of 16 column tiles (per-tile kernel),
+    # The same columns in launches of 16 column tiles,
     # reading B and writing D in place through offsets (ldb = ldd = N).
     P = torch.full_like(D, float("nan"))
     for c0 in list(range(0, min(N, 4 * 16 * BN), 16 * BN)) + [N - 16 * BN]:
@@ -467,28 +512,29 @@ def test_gemm_persistent_matches_per_tile_kernel(hip, dt, M, ntiles, K, batch, a
 @pytest.mark.parametrize("alpha,beta,with_c", [(1.0, 0.0, False), (1.5, 0.5, True)])
 def test_gemm_small_tile_matches_wide_tiles(hip, dt, M, N, K, batch, alpha, beta, with_c):
     """M, N <= 32 with both operands k-contiguous and K within one deep stage
-    (config 1's 'ap,bp->ab', 32 x 32 x 96): the 32 x 32 single-stage tile.
-    Checked against float64 torch, and bitwise against the same outputs as
-    part of a wider problem (M = 40 takes the 64-row tiles; the extra rows
-    do not change the first M), which keeps the k order per output."""
+    (config 1's 'ap,bp->ab', 32 x 32 x 96): one 32 x 32 tile. Checked against
+    float64 torch, and bitwise against the same outputs as part of a 1000 x
+    2000 problem, which takes wide tiles (fp64 direct-B; fp32 64 x 128): the
+    extra rows and columns do not change the first, and the k order per output
+    is the same."""
     from trntensor_amd.hip import engine
 
     g = torch.Generator().manual_seed(M * 7 + N + K + batch)
     dev = torch.device("cuda")
-    Mw = 40
+    Mw, Nw = 1000, 2000
     A = torch.randn(batch, Mw, K, generator=g, dtype=torch.float64)
-    B = torch.randn(batch, N, K, generator=g, dtype=torch.float64)
-    C = torch.randn(batch, Mw, N, generator=g, dtype=torch.float64)
-    ref = alpha * torch.bmm(A[:, :M], B.transpose(1, 2).contiguous())
+    B = torch.randn(batch, Nw, K, generator=g, dtype=torch.float64)
+    C = torch.randn(batch, Mw, Nw, generator=g, dtype=torch.float64)
+    ref = alpha * torch.bmm(A[:, :M], B[:, :N].transpose(1, 2).contiguous())
     if with_c:
-        ref = ref + beta * C[:, :M]
+        ref = ref + beta * C[:, :M, :N]
     Ad, Bd, Cd = A.to(dev, dt), B.to(dev, dt), C.to(dev, dt)
     outs = []
-    for m in (M, Mw):
-        D = torch.full((batch, Mw, N), float("nan"), dtype=dt, device=dev)
-        engine.gemm(False, True, m, N, K, Ad, K, Mw * K, Bd, K, N * K, D, N, Mw * N, batch, alpha, beta,
-                    Cd if with_c else None, N, Mw * N)
-        outs.append(D[:, :M])
+    for m, n in ((M, N), (Mw, Nw)):
+        D = torch.full((batch, Mw, Nw), float("nan"), dtype=dt, device=dev)
+        engine.gemm(False, True, m, n, K, Ad, K, Mw * K, Bd, K, Nw * K, D, Nw, Mw * Nw, batch, alpha, beta,
+                    Cd if with_c else None, Nw, Mw * Nw)
+        outs.append(D[:, :M, :N])
     torch.cuda.synchronize()
     assert normwise(outs[0], ref) <= TOL[dt]
     assert torch.equal(outs[0], outs[1])
@@ -499,8 +545,8 @@ def test_gemm_big_tile_broadcast_b(hip, with_c):
     """fp32 batched products sharing one B (batch stride 0, the engine's
     broadcast of an unbatched operand), whole 256 x 256 tiles filling the
     chip: the 256 x 256 LDS tile (with C only for K >= 1024). Checked against
-    float64 torch, and bitwise against the LDS-staged tiles, which take the
-    same problem when B's leading dimension breaks 16-byte alignment."""
+    float64 torch, and bitwise against the 64 x 256 direct-B tiles, which take
+    the same problem when B's leading dimension breaks 16-byte alignment."""
     from trntensor_amd.hip import engine
 
     dev = torch.device("cuda")
@@ -515,7 +561,7 @@ def test_gemm_big_tile_broadcast_b(hip, with_c):
         ref = ref + 0.5 * C
     Ad, Cd = A.to(dev, torch.float32), C.to(dev, torch.float32)
     Bn = B[:, :N].contiguous().to(dev, torch.float32)  # ldb = N: the 256 x 256 tile
-    Bo = B.contiguous().to(dev, torch.float32)  # ldb = N + 1: the LDS-staged tiles
+    Bo = B.contiguous().to(dev, torch.float32)  # ldb = N + 1: the 64 x 256 direct-B tiles
     outs = []
     for Bd, ldb in ((Bn, N), (Bo, N + 1)):
         D = torch.full((batch, M, N), float("nan"), dtype=torch.float32, device=dev)

@@ -59,8 +59,8 @@ def test_mp2_fp32_matches_oracle(hip, shape):
     assert rel(got, ref) <= 1e-5
 
 
-# naux with rows not 16-byte aligned: fp32 even (8-byte loads), odd (4-byte
-# loads); fp64 odd (8-byte loads). Full and ragged virtual blocks.
+# naux with rows not 16-byte aligned (8 or 4 bytes), read in 16-byte pieces at
+# the element's alignment. Full and ragged virtual blocks.
 UNALIGNED = [
     (6, 130, 1190),
     (4, 70, 1199),
@@ -133,7 +133,7 @@ def test_mp2_row_padded_copy_is_bitwise_neutral(hip, shape, dtype, offset):
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
 def test_mp2_misaligned_base_pointer(hip, dtype):
     """B contiguous but starting one element past a 16-byte boundary (a view
-    into a larger buffer): the loads narrow to the base's alignment. The
+    into a larger buffer): 16-byte loads at the element's alignment. The
     energy equals the aligned copy's bitwise (same values, same order)."""
     nocc, nvir, naux = 5, 70, 64
     B, eo, ev = inputs(nocc, nvir, naux, dtype=dtype, seed=31)
