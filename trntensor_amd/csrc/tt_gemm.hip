@@ -1095,9 +1095,11 @@ static int gemm_f64(GemmArgs& g, bool ta, bool tb, hipStream_t st) {
     const int64_t cus = device_cus();
     auto up = [](int64_t n, int64_t t) { return (n + t - 1) / t; };
     // A wave past the last column does not give all of its share back where K is
-    // long: 292 x 9 x 190 x 199 (one live wave of four) 22 us on 64 rows, 31 on 32.
+    // long. us on 32 x 128 / 32 x 32: 284545 x 7 x 222 NT 170 / 119, 137622 x 9 x 302
+    // NT 104 / 75, 57 x 11 x 607 x 513 TN 55 / 43; but 34 x 19 x 447 x 1866 83 (48 rows)
+    // / 96.
     double cols = (double)(up(g.N, 32) * 32) / (double)(up(g.N, 128) * 128);
-    if (g.K > 32) cols = std::max(cols, 0.6);
+    if (g.K > 32) cols = std::max(cols, g.N <= 32 ? 0.4 : 0.55);
     auto direct = [&](int64_t fm, double per_output) {
         const int64_t n = up(g.M, 16 * fm) * up(g.N, 128) * g.batch;
         if (n > kMaxGrid) return 1e300;  // not one launch; the 32 x 32 tiles take several
