@@ -1431,14 +1431,24 @@ extern "C" int tt_gemm_dot(int dtype, int transA, int transB, int64_t M, int64_t
         // contiguous along n: 4065 x 21285 x 4 (10688 / 10656) 262 / 469, 1605 x 19235
         // x 12 124 / 175, 128 x 20254 x 533 80 / 85, 27541 x 256 x 270 84 / 99; but
         // 19486 x 773 x 417 (9 tiles on a CU / 8) 255 / 224, 16501 x 9 x 70 18 / 13.
-        auto dot_cost = [&](int64_t m, int64_t n, int lane) {
+        const int64_t given = ((M + 63) / 64) * ((N + 127) / 128) * batch;
+        const int64_t exch = ((N + 63) / 64) * ((M + 127) / 128) * batch;
+        auto pen = [&](int lane) {
             auto strided = [&](const int64_t* s) { return s[lane] > 16 || s[lane] < -16; };
-            const int64_t pen = strided(g.e1s) || (E2 && strided(g.e2s)) ? 50 : 0;
-            const int64_t tiles = ((m + 63) / 64) * ((n + 127) / 128) * batch, cus = device_cus();
-            if (tiles > 0x7fffffffLL) return 1e300;  // not launched
-            return (double)((tiles + cus - 1) / cus) * (double)(K + 60 + pen) + 1e-10 * (double)tiles;
+            return strided(g.e1s) || (E2 && strided(g.e2s)) ? 50 : 0;
         };
-        if (dtype == TT_F64 && dot_cost(N, M, m_lo > 1 ? 1 : 0) < dot_cost(M, N, n_lo > 1 ? 3 : 2)) {
+        bool exchange = false;
+        if (dtype == TT_F64 && exch <= 0x7fffffffLL) {
+            const int64_t kg = K + 60 + pen(n_lo > 1 ? 3 : 2), ke = K + 60 + pen(m_lo > 1 ? 1 : 0);
+            double cg = (double)kg, ce = (double)ke;
+            if (std::max(given, exch) > 64) {  // else one round of the CUs either way
+                const int64_t cus = device_cus();
+                cg *= (double)((given + cus - 1) / cus);
+                ce *= (double)((exch + cus - 1) / cus);
+            }
+            exchange = ce < cg || (ce == cg && exch < given);
+        }
+        if (exchange) {
             std::swap(g.A, g.B);
             std::swap(g.M, g.N);
             std::swap(g.lda, g.ldb);
