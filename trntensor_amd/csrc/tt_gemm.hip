@@ -78,6 +78,16 @@ __global__ __launch_bounds__(kThreads) void gemm_kernel(GemmArgs g) {
 
     SA sa;
     SB sb;
+    // The dot's few wide tiles often lie mostly past a ragged edge, and loading
+    // clamped pieces there costs more than the branch: us, fp32, loaded / skipped /
+    // under the guards before the clamped loads: 12288 x 72 x 892 NN 60 / 51 / 53, TT
+    // 59 / 49 / 54, 5352 x 128 x 1243 x 3 TN 87 / 71 / 82. Not with both operands
+    // k-contiguous (4100 x 4001 x 512 NT 201 / 251 / 204, 2000 x 3000 x 1001 117 / 130).
+    constexpr bool SKIP = DOT && !FULL && (TA || !TB);
+    if constexpr (SKIP) {
+        sa.clear();
+        sb.clear();
+    }
     const int64_t nk = (g.K + BK - 1) / BK;
     // Stages 0 .. nfull-1 have all their k in range (a row-contiguous operand
     // with fewer rows than one vector takes the guarded loads throughout).
@@ -86,8 +96,8 @@ __global__ __launch_bounds__(kThreads) void gemm_kernel(GemmArgs g) {
     // chose for 64-deep stages), they capture acc by reference and the
     // accumulators go to scratch memory.
     auto load = [&](int64_t k0) __attribute__((always_inline)) {
-        sa.template load<FULL>(A, g.lda, m0, g.M, k0);
-        sb.template load<FULL>(B, g.ldb, n0, g.N, k0);
+        sa.template load<FULL, SKIP>(A, g.lda, m0, g.M, k0);
+        sb.template load<FULL, SKIP>(B, g.ldb, n0, g.N, k0);
     };
     auto load_tail = [&](int64_t k0) __attribute__((always_inline)) {
         sa.load_tail(A, g.lda, m0, g.M, k0, g.K);

@@ -48,6 +48,13 @@ struct Stage {
 
     vec_t reg[NC];
 
+    __device__ __forceinline__ void clear() {
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int e = 0; e < V; ++e) reg[c][e] = T(0);
+    }
+
     __device__ __forceinline__ static void place(int& row, int& k) {
         const int t = threadIdx.x;
         if (KC) {
@@ -74,10 +81,14 @@ struct Stage {
     // and loaded element by element when unaligned, as before, the edge
     // tiles set the time of the launch (fp32 1999 x 3001 x 1201 with
     // alpha/beta and C, all odd: 150 us against 224).
-    template <bool INSIDE>
+    // SKIP: pieces wholly past the edge are not loaded and keep what the
+    // registers held (clear() them first), for kernels with tiles that lie mostly
+    // past it.
+    template <bool INSIDE, bool SKIP = false>
     __device__ __forceinline__ void load(const T* __restrict__ p, int64_t ld, int64_t row0, int64_t rows, int64_t k0) {
         int r, k;
         place(r, k);
+        if (!INSIDE && SKIP && KC && row0 + r >= rows) return;
         if (INSIDE || KC) {
             const int64_t row = INSIDE ? row0 + r : min(row0 + r, rows - 1);
             const T* src = KC ? p + row * ld + (k0 + k) : p + (k0 + k) * ld + row;
@@ -89,6 +100,7 @@ struct Stage {
         } else {
 #pragma unroll
             for (int c = 0; c < NC; ++c) {
+                if (SKIP && row0 + r + prow(c) >= rows) continue;
                 const int64_t row = min(row0 + r + prow(c), rows - V);
                 const mem_t* q = reinterpret_cast<const mem_t*>(p + (k0 + k + pk(c)) * ld + row);
                 reg[c] = *q;
