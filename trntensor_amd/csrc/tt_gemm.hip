@@ -1110,12 +1110,18 @@ static int gemm_f64(GemmArgs& g, bool ta, bool tb, hipStream_t st) {
     // / 96.
     double cols = (double)(up(g.N, 32) * 32) / (double)(up(g.N, 128) * 128);
     if (g.K > 32) cols = std::max(cols, g.N <= 32 ? 0.4 : 0.55);
+    // Few rows and a long k-contiguous B: a direct-B lane reads its own column's
+    // row, and nothing but the stage ahead covers that stream; the 32 x 32 tile
+    // stages whole lines. us on 64 / 48 / 32 rows / 32 x 32: 60 x 69201 x 282 92 / 140 /
+    // 119 / 59, 50 x 277167 x 330 403 / 702 / 638 / 276, 17 x 40746 x 654 105 / 101 / 97 /
+    // 45; up to K = 80 level (37 x 78114 x 63 26 / 21 / 27 / 30).
+    const double stream = tb && g.M <= 64 && g.K > 80 ? 1.5 : 1.0;
     auto direct = [&](int64_t fm, double per_output) {
         const int64_t n = up(g.M, 16 * fm) * up(g.N, 128) * g.batch;
         if (n > kMaxGrid) return 1e300;  // not one launch; the 32 x 32 tiles take several
         const int64_t rounds = up(n, cus);
         const double share = rounds == 1 ? 1.0 : rounds == 2 ? (1.0 + cols) / 2 : cols;
-        return (double)(rounds * 16 * fm * 128) * share * per_output * (rounds == 1 ? 1.6 : 1.0);
+        return (double)(rounds * 16 * fm * 128) * share * per_output * (rounds == 1 ? 1.6 : 1.0) * stream;
     };
     const int64_t sr = up(up(g.M, 32) * up(g.N, 32) * g.batch, cus);
     // A short sum leaves most of a 64-deep stage empty: 318 x 3602 x 7 NT 7.7 us
